@@ -126,6 +126,33 @@ def test_gemm_quant_bitwise(gpu, t, in_dim, out_dim, tokens):
         assert same_floats(got, fo.ref_gemm(t, w, x, out_dim, in_dim))
 
 
+@pytest.mark.parametrize("t,in_dim,out_dim,tokens", [
+    # whole stages of 64 columns, one past and one short; 32- and 64-token
+    # tiles, full and with one row; fewer stages than are requested ahead
+    (0, 64, 33, 64), (0, 72, 32, 65), (0, 327, 5, 33), (0, 448, 31, 2), (8, 64, 31, 32), (8, 352, 65, 96),
+    (2, 32, 64, 33), (2, 640, 33, 64), (12, 1280, 32, 65), (14, 768, 31, 31)])
+def test_gemm_quant_tile_edges_bitwise(gpu, t, in_dim, out_dim, tokens):
+    """Tile and stage edges of the matrix-core product, bit for bit. The last
+    token's products all underflow to -0 where the row is negative, so that
+    padding which added +0 anywhere would show in the sign."""
+    import torch
+    rng = np.random.default_rng(in_dim * 7 + out_dim * 3 + tokens + t)
+    w = wl.matrix(t, rng, out_dim, in_dim, sigma=0.03, f32_sigma=0.3)
+    x = rng.standard_normal((tokens, in_dim), dtype=np.float32)
+    if t == 0:
+        w.view(np.float32)[-1] = np.clip(-np.abs(w.view(np.float32)[-1]), -0.4, -0.01)
+    x[-1] = np.float32(1e-45)
+    y = torch.full((tokens, out_dim), float("nan"), dtype=torch.float32, device=gpu)
+    wd, xd = dev(w, gpu), dev(x, gpu)
+    fmx.call("fmx_gemm_quant", t, wd.data_ptr(), xd.data_ptr(), y.data_ptr(), tokens, out_dim, in_dim,
+             fmx.stream_handle())
+    torch.cuda.synchronize()
+    got, want = y.cpu().numpy(), fo.gemm(t, w, x, out_dim, in_dim)
+    assert same_floats(got, want)
+    if t == 0:
+        assert np.signbit(want[-1, -1]) and want[-1, -1] == 0.0
+
+
 def test_gemm_quant_errors(gpu):
     """The reference's argument checks: a zero dimension is a no-op, a row that
     is not whole blocks is SHAPE_MISMATCH, an unknown type UNSUPPORTED."""

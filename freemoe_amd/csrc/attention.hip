@@ -16,104 +16,526 @@
 // on a rounding boundary. A non-finite score (the engine raises
 // INTERNAL_ERROR) sets bit 0 of the status word.
 //
-// One workgroup per query head: the head's scores and exponentials stay in
-// LDS (positions <= kMaxPositions), one lane adds the exponentials in order,
-// and head_dim lanes run the value sums.
+// Both sums over the positions are formed in parallel with a bound on how far
+// the sum in position order can lie from the parallel one. A probability or
+// an output whose float is the same over that whole interval is the engine's;
+// where one is not, one lane adds the terms in order. For 32 heads of 128 over
+// 8 kv heads and 2000 positions (16 MB of cache: 3 us of HBM) a call takes 20
+// us, three dependent launches of 1, 5 and 11 us, each a chain of memory,
+// LDS and double-precision latencies; walking every sum in order on one
+// workgroup per head took 215 us (32 of the 256 CUs in use). 8192 positions:
+// 50-67 us.
+#include <atomic>
+
 #include "fmx_internal.hpp"
 
 namespace fmx {
 
 namespace {
 
-constexpr uint32_t kAttnThreads = 256;
 constexpr uint32_t kMaxHeadDim = 256;
 constexpr uint32_t kMaxPositions = 8192;
+constexpr uint32_t kScorePos = 32;  // positions of a score workgroup
+constexpr uint32_t kScoreHeads = 4; // heads it scores at a time
+constexpr uint32_t kSliceDims = 16; // output elements of a value workgroup
+constexpr uint32_t kGroupPad = 4;   // its LDS rows of group sums: the four columns' stores on other banks
 
-__device__ inline float block_max(float v, float *red) {
-    for (uint32_t m = 32; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m));
-    const uint32_t w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) red[w] = v;
-    __syncthreads();
-    float r = red[0];
-    for (uint32_t i = 1; i < kAttnThreads / 64; ++i) r = fmaxf(r, red[i]);
-    __syncthreads();
-    return r;
+// Up to this many positions every slice's workgroup computes the scores of its
+// head itself, one per thread: 32 heads of 128 over 256 positions 11.7 against
+// 15.3 us with the score kernel's launch before it (at 512, two per thread,
+// no faster).
+constexpr uint32_t kSplitPositions = 256;
+
+// Scores between the two kernels of a call: slots of device memory, taken and
+// given back on the device. A call's ticket names its slot; the slot is the
+// call's where attention_begin_kernel found it free, until the call's last
+// value workgroup frees it. A call that found its slot taken (more than kSlots
+// calls in flight, or a replayed graph's fixed ticket meeting another call's)
+// computes the scores in the value kernel. (Taking it in every score
+// workgroup instead saves that launch, 2 us, but its atomics on one address
+// cost 10 ns each: the score kernel 5.8 -> 15.7 us for 504 workgroups.)
+constexpr uint32_t kSlots = 8;
+constexpr uint32_t kSlotFloats = 512 * 1024;
+__device__ __align__(256) float slot_scores[kSlots][kSlotFloats];
+struct Slot {
+    uint32_t owner; // ticket, 0: free
+    uint32_t done;  // value workgroups past their reads
+    uint32_t pad[62];
+};
+__device__ Slot slots[kSlots];
+
+__device__ __forceinline__ bool owns_slot(uint32_t ticket) {
+    return ticket != 0 && slots[ticket % kSlots].owner == ticket;
 }
 
-// grid: heads; LDS: positions floats (scores, then probabilities) and
-// positions doubles (exponentials).
-__global__ __launch_bounds__(kAttnThreads) void attention_decode_kernel(
-    const float *__restrict__ q, const float *__restrict__ kv, uint64_t row_stride, uint32_t v_offset,
-    uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t positions, double scale,
-    float *__restrict__ out, uint32_t *__restrict__ status) {
-    extern __shared__ __align__(16) char lds[];
-    __shared__ __align__(16) float qs[kMaxHeadDim];
-    __shared__ float red[kAttnThreads / 64];
-    __shared__ double sum_s;
-    __shared__ int bad_s;
-    float *sc = reinterpret_cast<float *>(lds);
-    double *ex = reinterpret_cast<double *>(lds + ((positions * 4 + 15) & ~15u));
-    const uint32_t tid = threadIdx.x, head = blockIdx.x;
-    const uint32_t kvh = head / (heads / kv_heads);
-    const uint32_t D = head_dim, D4 = D / 4;
-    for (uint32_t j = tid; j < D; j += kAttnThreads) qs[j] = q[static_cast<uint64_t>(head) * D + j];
-    if (tid == 0) bad_s = 0;
-    __syncthreads();
-    // scores: one position per thread, its key read as float4s
-    bool bad = false;
-    for (uint32_t t = tid; t < positions; t += kAttnThreads) {
-        const float4 *k4 = reinterpret_cast<const float4 *>(kv + t * row_stride + static_cast<uint64_t>(kvh) * D);
-        double dot = 0.0;
-        for (uint32_t j4 = 0; j4 < D4; ++j4) {
-            const float4 k = k4[j4];
-            dot += static_cast<double>(qs[4 * j4]) * static_cast<double>(k.x);
-            dot += static_cast<double>(qs[4 * j4 + 1]) * static_cast<double>(k.y);
-            dot += static_cast<double>(qs[4 * j4 + 2]) * static_cast<double>(k.z);
-            dot += static_cast<double>(qs[4 * j4 + 3]) * static_cast<double>(k.w);
-        }
-        const float s = static_cast<float>(dot * scale);
-        bad |= !__builtin_isfinite(s);
-        sc[t] = s;
+__global__ void attention_begin_kernel(uint32_t *status, uint32_t ticket) {
+    *status = 0;
+    if (ticket != 0 && atomicCAS(&slots[ticket % kSlots].owner, 0u, ticket) == 0u) slots[ticket % kSlots].done = 0;
+}
+
+// The dot of one key with one query (doubles in LDS), in index order. fma:
+// the product is exact, so it rounds once, as the engine's multiply and add.
+__device__ __forceinline__ double dot_in_order(const float *k, const double *q, uint32_t head_dim) {
+    double dot = 0.0;
+#pragma unroll 8
+    for (uint32_t j = 0; j < head_dim; j += 4) {
+        const float4 v = *reinterpret_cast<const float4 *>(k + j);
+        const double2 a = *reinterpret_cast<const double2 *>(q + j);
+        const double2 b = *reinterpret_cast<const double2 *>(q + j + 2);
+        dot = fma(a.x, static_cast<double>(v.x), dot);
+        dot = fma(a.y, static_cast<double>(v.y), dot);
+        dot = fma(b.x, static_cast<double>(v.z), dot);
+        dot = fma(b.y, static_cast<double>(v.w), dot);
     }
-    if (__any(bad) && (tid & 63) == 0) bad_s = 1;
+    return dot;
+}
+
+// Scores of 32 positions for every query head of one kv head, into the call's
+// slot. The keys are read once, whole rows at a time, into LDS (rows 4 floats
+// apart in banks); a lane runs one (position, head) chain of head_dim fmas.
+// grid: position tiles x kv heads; LDS: keys, then 4 heads' queries.
+__global__ __launch_bounds__(kScorePos *kScoreHeads) void attention_scores_kernel(
+    const float *__restrict__ q, const float *__restrict__ kv, uint64_t row_stride, uint32_t group,
+    uint32_t head_dim, uint32_t positions, double scale, uint32_t ticket) {
+    extern __shared__ __align__(16) char lds[];
+    __shared__ bool own_s;
+    if (threadIdx.x == 0) own_s = owns_slot(ticket);
+    const uint32_t tid = threadIdx.x, kvh = blockIdx.y, t0 = blockIdx.x * kScorePos;
+    const uint32_t kstride = head_dim + 4, qstride = head_dim + 2, D4 = head_dim / 4;
+    float *ks = reinterpret_cast<float *>(lds);
+    double *qs = reinterpret_cast<double *>(ks + kScorePos * kstride);
+    const float *keys = kv + static_cast<uint64_t>(kvh) * head_dim;
+#pragma unroll 8
+    for (uint32_t i = tid; i < kScorePos * D4; i += kScorePos * kScoreHeads) {
+        const uint32_t p = i / D4, j = i % D4;
+        const uint32_t t = t0 + p < positions ? t0 + p : positions - 1; // clamp: loads stay in the cache
+        *reinterpret_cast<float4 *>(ks + p * kstride + 4 * j) =
+            *reinterpret_cast<const float4 *>(keys + t * row_stride + 4 * j);
+    }
+    const uint32_t pos = tid % kScorePos, hs = tid / kScorePos;
+    float *dst = slot_scores[ticket % kSlots] + t0 + pos;
+    for (uint32_t h0 = 0; h0 < group; h0 += kScoreHeads) {
+        const uint32_t nh = group - h0 < kScoreHeads ? group - h0 : kScoreHeads;
+        const uint64_t head0 = static_cast<uint64_t>(kvh) * group + h0;
+        if (h0) __syncthreads();
+        for (uint32_t i = tid; i < nh * head_dim; i += kScorePos * kScoreHeads)
+            qs[i / head_dim * qstride + i % head_dim] = static_cast<double>(q[head0 * head_dim + i]);
+        __syncthreads();
+        if (!own_s) return;
+        if (hs < nh && t0 + pos < positions)
+            dst[(head0 + hs) * positions] =
+                static_cast<float>(dot_in_order(ks + pos * kstride, qs + hs * qstride, head_dim) * scale);
+    }
+}
+
+// v moved across lanes by one DPP step; 0 where the step has no source lane.
+template <int kCtrl, int kRows>
+__device__ __forceinline__ double dpp_or_zero(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), kCtrl, kRows, 0xF, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), kCtrl, kRows, 0xF, true);
+    return __builtin_bit_cast(double, static_cast<uint64_t>(hi) << 32 | lo);
+}
+
+// Inclusive sum over the lanes of a wavefront: row_shr:1, 2, 4, 8 inside the
+// rows of 16, then lane 15 of each even row into the odd row after it, then
+// lane 31 into the upper half.
+__device__ __forceinline__ double wave_scan(double v) {
+    v += dpp_or_zero<0x111, 0xF>(v);
+    v += dpp_or_zero<0x112, 0xF>(v);
+    v += dpp_or_zero<0x114, 0xF>(v);
+    v += dpp_or_zero<0x118, 0xF>(v);
+    v += dpp_or_zero<0x142, 0xA>(v);
+    v += dpp_or_zero<0x143, 0xC>(v);
+    return v;
+}
+
+__device__ __forceinline__ double last_lane(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = __builtin_amdgcn_readlane(static_cast<int>(b), 63);
+    const uint32_t hi = __builtin_amdgcn_readlane(static_cast<int>(b >> 32), 63);
+    return __builtin_bit_cast(double, static_cast<uint64_t>(hi) << 32 | lo);
+}
+
+__device__ __forceinline__ double wave_sum(double v) { return last_lane(wave_scan(v)); }
+
+// s + a[0] + a[1] + ... in order, for one lane: the next 16 terms are read
+// from LDS during the current 16's additions.
+__device__ __forceinline__ double add_in_order(const double *a, uint32_t n, double s) {
+    constexpr uint32_t kBatch = 16;
+    double cur[kBatch], next[kBatch];
+    const uint32_t full = n / kBatch * kBatch;
+    if (full) {
+#pragma unroll
+        for (uint32_t i = 0; i < kBatch; ++i) cur[i] = a[i];
+    }
+    for (uint32_t t = 0; t < full; t += kBatch) {
+        const double *from = a + (t + kBatch < full ? t + kBatch : t);
+#pragma unroll
+        for (uint32_t i = 0; i < kBatch; ++i) next[i] = from[i];
+#pragma unroll
+        for (uint32_t i = 0; i < kBatch; ++i) s += cur[i];
+#pragma unroll
+        for (uint32_t i = 0; i < kBatch; ++i) cur[i] = next[i];
+    }
+    for (uint32_t t = full; t < n; ++t) s += a[t];
+    return s;
+}
+
+__device__ __forceinline__ uint32_t exponent_of(double v) {
+    return static_cast<uint32_t>(__builtin_bit_cast(uint64_t, v) >> 52);
+}
+__device__ __forceinline__ double power_of(uint32_t exponent) { // 0 below the normal range
+    return __builtin_bit_cast(double, static_cast<uint64_t>(exponent) << 52);
+}
+
+// hi + lo += v, exactly but for the last rounding of lo.
+__device__ __forceinline__ void add_exact(double &hi, double &lo, double v, double v_lo = 0.0) {
+    const double s = hi + v, b = s - hi;
+    lo += ((hi - (s - b)) + (v - b)) + v_lo;
+    hi = s;
+}
+
+// The sum of a workgroup's terms in order, s_t = rn(s_t-1 + x_t) from 0, to
+// within `doubt`: thread i holds the nt <= kTerms terms after thread i - 1's
+// and the (unordered) sum `run` of those before, which no ordered prefix sum
+// is further from than `margin`. While s stays in one binade, of unit u, a
+// step adds x_t rounded to a multiple of u, whatever s is, but for exact ties;
+// so where the margin leaves no doubt about the binades of s_t-1 and s_t, the
+// step is known but for half a unit at a tie, and elsewhere to within a unit.
+// Every thread returns the same sum; red: 3 x kWaves doubles of LDS. x_t has
+// at most 48 significant bits or is no larger in magnitude than s_t.
+template <uint32_t kTerms, uint32_t kWaves>
+__device__ __forceinline__ void ordered_interval(const double (&x)[kTerms], uint32_t nt, double run, double margin,
+                                                 double (&red)[3][kWaves], double &sum, double &doubt) {
+    double hi = 0.0, lo = 0.0, unc = 0.0;
+#pragma unroll
+    for (uint32_t i = 0; i < kTerms; ++i)
+        if (i < nt) {
+            const double after = run + x[i];
+            const uint32_t k = exponent_of(fabs(after) + margin);
+            const double u = power_of(k > 52 ? k - 52 : 0);
+            double r = x[i];
+            if (exponent_of(fabs(after) - margin) != k || fabs(run) <= margin || exponent_of(fabs(run) - margin) < k) {
+                unc += u;
+            } else if (fabs(x[i]) < power_of(k)) { // else a multiple of u
+                const double big = copysign(power_of(k), x[i]);
+                r = (big + x[i]) - big;
+                if (fabs(x[i] - r) * 2.0 == u) {
+                    r = x[i];
+                    unc += 0.5 * u;
+                }
+            }
+            add_exact(hi, lo, r);
+            run = after;
+        }
+    auto wave_total = [&] {
+        add_exact(hi, lo, dpp_or_zero<0x111, 0xF>(hi), dpp_or_zero<0x111, 0xF>(lo));
+        add_exact(hi, lo, dpp_or_zero<0x112, 0xF>(hi), dpp_or_zero<0x112, 0xF>(lo));
+        add_exact(hi, lo, dpp_or_zero<0x114, 0xF>(hi), dpp_or_zero<0x114, 0xF>(lo));
+        add_exact(hi, lo, dpp_or_zero<0x118, 0xF>(hi), dpp_or_zero<0x118, 0xF>(lo));
+        add_exact(hi, lo, dpp_or_zero<0x142, 0xA>(hi), dpp_or_zero<0x142, 0xA>(lo));
+        add_exact(hi, lo, dpp_or_zero<0x143, 0xC>(hi), dpp_or_zero<0x143, 0xC>(lo));
+        hi = last_lane(hi);
+        lo = last_lane(lo);
+        unc = wave_sum(unc);
+    };
+    wave_total();
+    const uint32_t lane = threadIdx.x & 63;
+    if (lane == 0) {
+        red[0][threadIdx.x >> 6] = hi;
+        red[1][threadIdx.x >> 6] = lo;
+        red[2][threadIdx.x >> 6] = unc;
+    }
     __syncthreads();
-    if (bad_s) {
-        if (tid == 0) atomicOr(status, STATUS_NONFINITE_SCORE);
-        for (uint32_t j = tid; j < D; j += kAttnThreads) out[static_cast<uint64_t>(head) * D + j] = 0.0f;
-        return;
+    hi = lane < kWaves ? red[0][lane] : 0.0;
+    lo = lane < kWaves ? red[1][lane] : 0.0;
+    unc = lane < kWaves ? red[2][lane] : 0.0;
+    wave_total();
+    sum = hi + lo;
+    // the bound's own roundings, and the sum's
+    doubt = unc * 1.0009765625 + fabs(sum) * 0x1p-52 + margin * 0x1p-40;
+}
+
+// grid: heads x slices of 16 output elements. LDS: positions doubles (the
+// exponentials where they are added in order; otherwise the probabilities as
+// floats), then the value sums of NT / 4 position groups.
+//
+// Softmax: every slice's workgroup repeats its head's, on NT threads of up to
+// kTerms consecutive positions. The sum of the exponentials in order is known
+// to a few units in 2^53 (ordered_interval), so all but about one of 2^23
+// probabilities are decided.
+//
+// Values: thread (g, c) sums its group's consecutive positions for four
+// elements; the sum in position order differs from theirs by at most the
+// roundings of its partial sums, each bounded by the prefix of the group it
+// is in plus the group's absolute sum. That decides all but about one of 10^5
+// elements (at 2000 positions; one of 10^4 at 8192); ordered_interval over
+// the element's products nearly all of the rest.
+template <uint32_t NT, uint32_t kTerms>
+__global__ __launch_bounds__(NT) void attention_values_kernel(
+    const float *__restrict__ q, const float *__restrict__ kv, uint64_t row_stride, uint32_t v_offset,
+    uint32_t heads, uint32_t group, uint32_t head_dim, uint32_t positions, double scale, float *__restrict__ out,
+    uint32_t *__restrict__ status, uint32_t ticket) {
+    constexpr uint32_t kWaves = NT / 64, kGroups = NT / (kSliceDims / 4), kPrefetch = 8;
+    constexpr uint32_t kGroupStride = kGroups + kGroupPad;
+    extern __shared__ __align__(16) char lds[];
+    __shared__ __align__(16) double qs[kMaxHeadDim];
+    __shared__ float red_max[kWaves];
+    __shared__ double red_sum[kWaves], red[3][kWaves], err_s[kSliceDims];
+    __shared__ bool own_s;
+    __shared__ uint32_t flags_s, todo_s; // 1: non-finite score, 2: a probability undecided
+    __shared__ double sum_s;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t P = positions, D = head_dim;
+    const uint32_t slices = div_up(D, kSliceDims), total = heads * slices;
+    // workgroup i runs on XCD i % 8: give each XCD consecutive heads, so that
+    // the heads of a kv head read its values through one L2
+    const uint32_t unit = total % 8 == 0 ? blockIdx.x % 8 * (total / 8) + blockIdx.x / 8 : blockIdx.x;
+    const uint32_t head = unit / slices, slice = unit % slices, kvh = head / group;
+    double *ex = reinterpret_cast<double *>(lds);
+    float *pr = reinterpret_cast<float *>(lds);
+    double *gsum = reinterpret_cast<double *>(lds + ((static_cast<size_t>(P) * 8 + 15) & ~static_cast<size_t>(15)));
+    float *gabs = reinterpret_cast<float *>(gsum + kSliceDims * kGroupStride);
+
+    // the first positions of this thread's values, in flight during the softmax
+    const uint32_t col = slice * kSliceDims + (tid & 3) * 4, grp = tid >> 2;
+    const uint32_t per_group = div_up(P, kGroups);
+    const uint32_t v0 = grp * per_group < P ? grp * per_group : P;
+    const uint32_t v1 = v0 + per_group < P ? v0 + per_group : P;
+    const float *vbase = kv + v_offset + static_cast<uint64_t>(kvh) * D + (col < D ? col : 0);
+    float4 vv[kPrefetch];
+#pragma unroll
+    for (uint32_t i = 0; i < kPrefetch; ++i) {
+        const uint32_t t = v0 + i < P ? v0 + i : P - 1;
+        vv[i] = *reinterpret_cast<const float4 *>(vbase + t * row_stride);
+    }
+
+    // scores t0 .. t1 - 1 of this thread
+    const uint32_t per = div_up(P, NT);
+    const uint32_t t0 = tid * per < P ? tid * per : P;
+    const uint32_t nt = t0 + per < P ? per : P - t0;
+    if (tid == 0) {
+        flags_s = todo_s = 0;
+        own_s = owns_slot(ticket);
+    }
+    __syncthreads();
+    const bool own = own_s;
+    float sc[kTerms];
+    if (own) {
+        const float *src = slot_scores[ticket % kSlots] + static_cast<uint64_t>(head) * P + t0;
+#pragma unroll
+        for (uint32_t i = 0; i < kTerms; ++i)
+            if (i < nt) sc[i] = src[i];
+    } else {
+        for (uint32_t j = tid; j < D; j += NT) qs[j] = static_cast<double>(q[static_cast<uint64_t>(head) * D + j]);
+        __syncthreads();
+#pragma unroll
+        for (uint32_t i = 0; i < kTerms; ++i)
+            if (i < nt)
+                sc[i] = static_cast<float>(
+                    dot_in_order(kv + (t0 + i) * row_stride + static_cast<uint64_t>(kvh) * D, qs, D) * scale);
     }
     float m = -__builtin_inff();
-    for (uint32_t t = tid; t < positions; t += kAttnThreads) m = fmaxf(m, sc[t]);
-    m = block_max(m, red);
-    const double md = static_cast<double>(m);
-    for (uint32_t t = tid; t < positions; t += kAttnThreads) ex[t] = exp(static_cast<double>(sc[t]) - md);
+    bool bad = false;
+#pragma unroll
+    for (uint32_t i = 0; i < kTerms; ++i)
+        if (i < nt) {
+            bad |= !__builtin_isfinite(sc[i]);
+            m = fmaxf(m, sc[i]);
+        }
+    for (uint32_t d = 32; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
+    if (lane == 0) red_max[wave] = m;
     __syncthreads();
-    if (tid == 0) {
-        double s = 0.0;
-        for (uint32_t t = 0; t < positions; ++t) s += ex[t];
-        sum_s = s;
+    if (__any(bad) && lane == 0) atomicOr(&flags_s, 1u);
+#pragma unroll
+    for (uint32_t i = 0; i < kWaves; ++i) m = fmaxf(m, red_max[i]);
+    const double md = static_cast<double>(m);
+    double e[kTerms], local = 0.0;
+#pragma unroll
+    for (uint32_t i = 0; i < kTerms; ++i) {
+        e[i] = i < nt ? exp(static_cast<double>(sc[i]) - md) : 0.0;
+        local += e[i];
+    }
+    const double incl = wave_scan(local);
+    if (lane == 63) red_sum[wave] = incl;
+    __syncthreads();
+    // every score of the head has reached its thread: the slot is read. (What
+    // takes it next starts after the exchange, so counting orders nothing: a
+    // release here would write back the L2.)
+    if (own && tid == 0 && atomicAdd(&slots[ticket % kSlots].done, 1u) + 1 == total)
+        atomicExch(&slots[ticket % kSlots].owner, 0u);
+    if (flags_s & 1u) {
+        if (tid == 0 && slice == 0) atomicOr(status, STATUS_NONFINITE_SCORE);
+        if (tid < 4 && col < D)
+            *reinterpret_cast<float4 *>(out + static_cast<uint64_t>(head) * D + col) = make_float4(0.f, 0.f, 0.f, 0.f);
+        return;
+    }
+    double run = incl - local, all = 0.0;
+#pragma unroll
+    for (uint32_t i = 0; i < kWaves; ++i) {
+        run += i < wave ? red_sum[i] : 0.0;
+        all += red_sum[i];
+    }
+    // (an ordered prefix sum is off by at most P 2^-53 of the whole, run by
+    // 30 2^-53)
+    double sum, doubt;
+    ordered_interval(e, nt, run, all * 0x1p-38, red, sum, doubt);
+    // relative: the doubt, the roundings of the reciprocal, of the products
+    // below and of the engine's division
+    const double rinv = 1.0 / sum, rel = doubt * rinv * 1.0009765625 + 0x1p-50;
+    float p[kTerms];
+    bool undecided = !(rel < 0x1p-30);
+#pragma unroll
+    for (uint32_t i = 0; i < kTerms; ++i)
+        if (i < nt) {
+            const double v = e[i] * rinv;
+            p[i] = static_cast<float>(v - v * rel);
+            undecided |= p[i] != static_cast<float>(v + v * rel);
+        }
+    if (__any(undecided) && lane == 0) atomicOr(&flags_s, 2u);
+    __syncthreads();
+    if (flags_s & 2u) { // the exponentials added in order by one lane
+#pragma unroll
+        for (uint32_t i = 0; i < kTerms; ++i)
+            if (i < nt) ex[t0 + i] = e[i];
+        __syncthreads();
+        if (tid == 0) sum_s = add_in_order(ex, P, 0.0);
+        __syncthreads();
+        const double s = sum_s;
+#pragma unroll
+        for (uint32_t i = 0; i < kTerms; ++i)
+            if (i < nt) p[i] = static_cast<float>(e[i] / s);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kTerms; ++i)
+        if (i < nt) pr[t0 + i] = p[i];
+    __syncthreads();
+
+    // values: this thread's positions of its group, four elements
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    float aabs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t tb = v0; tb < v1; tb += kPrefetch) {
+        float4 cur[kPrefetch];
+#pragma unroll
+        for (uint32_t i = 0; i < kPrefetch; ++i) {
+            cur[i] = vv[i];
+            const uint32_t t = tb + kPrefetch + i < P ? tb + kPrefetch + i : P - 1;
+            if (tb + kPrefetch < v1) vv[i] = *reinterpret_cast<const float4 *>(vbase + t * row_stride);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < kPrefetch; ++i)
+            if (tb + i < v1) {
+                const float w = pr[tb + i];
+                const double wd = static_cast<double>(w);
+                const float x[4] = {cur[i].x, cur[i].y, cur[i].z, cur[i].w};
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    acc[j] = fma(wd, static_cast<double>(x[j]), acc[j]);
+                    aabs[j] = fma_rn(w, fabsf(x[j]), aabs[j]);
+                }
+            }
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+        gsum[((tid & 3) * 4 + j) * kGroupStride + grp] = acc[j];
+        gabs[((tid & 3) * 4 + j) * kGroupStride + grp] = aabs[j];
     }
     __syncthreads();
-    const double sum = sum_s;
-    for (uint32_t t = tid; t < positions; t += kAttnThreads) sc[t] = static_cast<float>(ex[t] / sum);
+    // a wavefront takes kPerWave elements: prefix sums of the groups and the bound
+    constexpr uint32_t kPerLane = kGroups / 64, kPerWave = kSliceDims / kWaves;
+#pragma unroll
+    for (uint32_t i = 0; i < kPerWave; ++i) {
+        const uint32_t d = wave * kPerWave + i;
+        double gs[kPerLane], ga[kPerLane], s = 0.0, a = 0.0;
+#pragma unroll
+        for (uint32_t k = 0; k < kPerLane; ++k) {
+            gs[k] = gsum[d * kGroupStride + lane * kPerLane + k];
+            // (the float sum's own error, and products below float's range)
+            ga[k] = static_cast<double>(gabs[d * kGroupStride + lane * kPerLane + k]) * 1.0009765625 + 0x1p-120;
+            s += gs[k];
+            a += ga[k];
+        }
+        const double scan = wave_scan(s);
+        double before = scan - s, bound = 0.0;
+#pragma unroll
+        for (uint32_t k = 0; k < kPerLane; ++k) {
+            bound += fabs(before) + ga[k];
+            before += gs[k];
+        }
+        // per_group roundings of partial sums no larger than |before| + ga,
+        // as many here of sums no larger than ga, and the tree's (of at most
+        // a each): each 2^-53 of its sum, and a sixteenth for the bounds' own
+        // roundings
+        const double value = last_lane(scan);
+        const double err = wave_sum(per_group * (bound + a) + 16.0 * a) * 0x1.1p-53;
+        const float lo = static_cast<float>(value - err), hi = static_cast<float>(value + err);
+        const uint32_t j = slice * kSliceDims + d;
+        if (lane == 0 && j < D) {
+            if (__builtin_bit_cast(uint32_t, lo) == __builtin_bit_cast(uint32_t, hi) && __builtin_isfinite(lo))
+                out[static_cast<uint64_t>(head) * D + j] = lo;
+            else {
+                atomicOr(&todo_s, 1u << d);
+                err_s[d] = err;
+            }
+        }
+    }
     __syncthreads();
-    // values: one output element per thread, positions in order
-    for (uint32_t j = tid; j < D; j += kAttnThreads) {
+    // the elements left: by the intervals of their products (exact in
+    // double), then in position order, the products in LDS and one lane adding
+    constexpr uint32_t kTile = kSliceDims * kGroupStride;
+    for (uint32_t todo = todo_s; todo; todo &= todo - 1) {
+        const uint32_t d = __builtin_ctz(todo), j = slice * kSliceDims + d;
         const float *v = kv + v_offset + static_cast<uint64_t>(kvh) * D + j;
-        double acc = 0.0;
-        for (uint32_t t = 0; t < positions; ++t)
-            acc += static_cast<double>(sc[t]) * static_cast<double>(v[t * row_stride]);
-        out[static_cast<uint64_t>(head) * D + j] = static_cast<float>(acc);
+        double x[kTerms], before = 0.0;
+#pragma unroll
+        for (uint32_t i = 0; i < kTerms; ++i) {
+            x[i] = i < nt ? static_cast<double>(p[i]) * static_cast<double>(v[(t0 + i) * row_stride]) : 0.0;
+            before += x[i];
+        }
+        const double mine = before, scan = wave_scan(mine);
+        if (lane == 63) red_sum[wave] = scan;
+        __syncthreads();
+        before = scan - mine;
+#pragma unroll
+        for (uint32_t i = 0; i < kWaves; ++i) before += i < wave ? red_sum[i] : 0.0;
+        // (err_s bounds the ordered sum's roundings and 17 2^-53 of the
+        // absolute sum; these prefixes' add up to 30 of them)
+        double s, off;
+        ordered_interval(x, nt, before, 3.0 * err_s[d], red, s, off);
+        const float lo = static_cast<float>(s - off), hi = static_cast<float>(s + off);
+        if (__builtin_bit_cast(uint32_t, lo) == __builtin_bit_cast(uint32_t, hi) && __builtin_isfinite(lo)) {
+            if (tid == 0) out[static_cast<uint64_t>(head) * D + j] = lo;
+            __syncthreads(); // red_sum and red are read
+            continue;
+        }
+        s = 0.0;
+        for (uint32_t tb = 0; tb < P; tb += kTile) {
+            const uint32_t n = P - tb < kTile ? P - tb : kTile;
+            for (uint32_t i = tid; i < n; i += NT)
+                gsum[i] = static_cast<double>(pr[tb + i]) * static_cast<double>(v[(tb + i) * row_stride]);
+            __syncthreads();
+            if (tid == 0) s = add_in_order(gsum, n, s);
+            __syncthreads();
+        }
+        if (tid == 0) out[static_cast<uint64_t>(head) * D + j] = static_cast<float>(s);
     }
 }
 
-__global__ void attention_clear_kernel(uint32_t *status) { *status = 0; }
+size_t values_lds_bytes(uint32_t positions, uint32_t threads) {
+    return ((static_cast<size_t>(positions) * 8 + 15) & ~static_cast<size_t>(15)) + (threads / 4 + kGroupPad) * kSliceDims * 12;
+}
+
+// Never 0; a call's slot is its ticket modulo kSlots.
+uint32_t next_ticket() {
+    static std::atomic<uint32_t> counter{0};
+    uint32_t t;
+    do t = counter.fetch_add(1, std::memory_order_relaxed) + 1;
+    while (t == 0);
+    return t;
+}
 
 } // namespace
-
-size_t attention_lds_bytes(uint32_t positions) {
-    return ((static_cast<size_t>(positions) * 4 + 15) & ~static_cast<size_t>(15)) + static_cast<size_t>(positions) * 8;
-}
 
 int attention_decode(const float *q, const float *kv, uint64_t row_stride, uint32_t v_offset, uint32_t heads,
                      uint32_t kv_heads, uint32_t head_dim, uint32_t positions, double scale, float *out,
@@ -124,12 +546,30 @@ int attention_decode(const float *q, const float *kv, uint64_t row_stride, uint3
     if (v_offset + static_cast<uint64_t>(kv_heads) * head_dim > row_stride ||
         static_cast<uint64_t>(kv_heads) * head_dim > v_offset)
         return FMX_ERR_SHAPE_MISMATCH;
-    const size_t lds = attention_lds_bytes(positions);
-    if (int rc = allow_lds(reinterpret_cast<const void *>(attention_decode_kernel), lds)) return rc;
-    hipLaunchKernelGGL(attention_clear_kernel, dim3(1), dim3(1), 0, s, status);
+    const uint32_t group = heads / kv_heads;
+    const uint32_t total = heads * div_up(head_dim, kSliceDims);
+    const bool split = positions > kSplitPositions && static_cast<uint64_t>(heads) * positions <= kSlotFloats &&
+                       kv_heads <= 65535;
+    const uint32_t ticket = split ? next_ticket() : 0;
+    // as few terms per thread as the threads allow: their exponentials and
+    // divisions are one after another
+    const auto values = positions <= 256    ? attention_values_kernel<256, 1>
+                        : positions <= 2048 ? attention_values_kernel<1024, 2>
+                                            : attention_values_kernel<1024, 8>;
+    const uint32_t threads = positions <= 256 ? 256 : 1024;
+    const size_t lds = values_lds_bytes(positions, threads);
+    if (int rc = allow_lds(reinterpret_cast<const void *>(values), lds)) return rc;
+    hipLaunchKernelGGL(attention_begin_kernel, dim3(1), dim3(1), 0, s, status, ticket);
     FMX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(attention_decode_kernel, dim3(heads), dim3(kAttnThreads), lds, s, q, kv, row_stride, v_offset,
-                       heads, kv_heads, head_dim, positions, scale, out, status);
+    if (split) {
+        const size_t tile = kScorePos * (head_dim + 4) * sizeof(float) + kScoreHeads * (head_dim + 2) * sizeof(double);
+        hipLaunchKernelGGL(attention_scores_kernel, dim3(div_up(positions, kScorePos), kv_heads),
+                           dim3(kScorePos * kScoreHeads), tile, s, q, kv, row_stride, group, head_dim, positions,
+                           scale, ticket);
+        FMX_LAUNCH_CHECK();
+    }
+    hipLaunchKernelGGL(values, dim3(total), dim3(threads), lds, s, q, kv, row_stride, v_offset, heads, group, head_dim,
+                       positions, scale, out, status, ticket);
     FMX_LAUNCH_CHECK();
     return FMX_OK;
 }

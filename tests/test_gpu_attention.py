@@ -83,3 +83,101 @@ def test_attention_decode_reports_nonfinite_scores(gpu):
     fmx.call("fmx_attention_decode", qd.data_ptr(), kvd.data_ptr(), 2 * kvh * D, kvh * D, heads, kvh, D, P, 0.5,
              out.data_ptr(), ws.data_ptr(), 256, fmx.stream_handle())
     assert fmx.lib().fmx_moe_status(ws.data_ptr(), fmx.stream_handle()) == 4  # FMX_ERR_INTERNAL
+
+
+ORDERED = {
+    # name: (heads, kv_heads, head_dim, positions): one and several slices and
+    # groups of four heads, ragged head dims, thread counts and their edges,
+    # scores in the value kernel and in the score kernel
+    "one": (1, 1, 4, 1),
+    "two": (3, 1, 36, 2),
+    "tile_edge_64": (8, 8, 64, 64),
+    "tile_edge_65": (10, 2, 64, 65),
+    "ragged_dim_997": (12, 2, 100, 997),
+    "wide_edge_1024": (8, 2, 96, 1024),
+    "wide_edge_1025": (8, 2, 96, 1025),
+    "gqa_32_of_8_2000": (32, 8, 128, 2000),
+    "mqa_6_of_1x256_4099": (6, 1, 256, 4099),
+    "longest_8192": (32, 32, 128, 8192),
+    "beyond_the_slot": (72, 8, 64, 8192),
+}
+
+
+def ordered_on_exp(q, kv, kv_heads, head_dim, v_offset, scale, gpu):
+    """reference() with the device's exp, so that every bit is determined."""
+    import torch
+    heads = q.shape[0] // head_dim
+    out = np.empty(heads * head_dim, np.float32)
+    for h in range(heads):
+        kvh = h // (heads // kv_heads)
+        qd = q[h * head_dim:(h + 1) * head_dim].astype(np.float64)
+        k = kv[:, kvh * head_dim:(kvh + 1) * head_dim].astype(np.float64)
+        s = (np.add.accumulate(k * qd, axis=1)[:, -1] * scale).astype(np.float32).astype(np.float64)
+        e = torch.exp(torch.from_numpy(s - s.max()).to(gpu)).cpu().numpy()
+        p = (e / np.add.accumulate(e)[-1]).astype(np.float32).astype(np.float64)
+        v = kv[:, v_offset + kvh * head_dim:v_offset + (kvh + 1) * head_dim].astype(np.float64)
+        with np.errstate(invalid="ignore"):
+            out[h * head_dim:(h + 1) * head_dim] = np.add.accumulate(p[:, None] * v, axis=0)[-1]
+    return out
+
+
+@pytest.mark.parametrize("spread", ["normal", "flat", "peaked"])
+@pytest.mark.parametrize("name", list(ORDERED))
+def test_attention_decode_keeps_the_ordered_sums(gpu, name, spread):
+    """Bit for bit the sums in position order, whichever of the certified and
+    the ordered way an element takes; cancelling, zero and infinite values,
+    and scores whose exponentials tie, lie far apart or are all alike."""
+    import torch
+    heads, kvh, D, P = ORDERED[name]
+    rng = np.random.default_rng(P * 31 + heads + len(spread))
+    kv_dim = kvh * D
+    kv = (rng.standard_normal((P, 2 * kv_dim)) * 0.5).astype(np.float32)
+    q = (rng.standard_normal(heads * D) * {"normal": 0.5, "flat": 0.0, "peaked": 6.0}[spread]).astype(np.float32)
+    kv[1::2, kv_dim] = -kv[:P - P % 2:2, kv_dim]  # element 0 cancels (where the weights allow)
+    kv[:, kv_dim + 1] = 0.0
+    kv[P // 2, kv_dim + 2] = np.inf
+    kv[:, kv_dim + 3] *= np.float32(1e-38)
+    scale = 1.0 / np.sqrt(float(D))
+    want = ordered_on_exp(q, kv, kvh, D, kv_dim, scale, gpu)
+    qd, kvd = torch.from_numpy(q).to(gpu), torch.from_numpy(kv).to(gpu)
+    ws = torch.zeros(256, dtype=torch.uint8, device=gpu)
+    for _ in range(2):
+        out = torch.full((heads * D,), 7.0, dtype=torch.float32, device=gpu)
+        fmx.call("fmx_attention_decode", qd.data_ptr(), kvd.data_ptr(), 2 * kv_dim, kv_dim, heads, kvh, D, P, scale,
+                 out.data_ptr(), ws.data_ptr(), 256, fmx.stream_handle())
+        assert fmx.lib().fmx_moe_status(ws.data_ptr(), fmx.stream_handle()) == 0
+        assert np.array_equal(out.cpu().numpy(), want, equal_nan=True)
+
+
+def test_attention_decode_calls_in_flight_share_no_scores(gpu):
+    """More calls in flight than the library holds score buffers, on streams
+    of their own, each with its own inputs and workspace."""
+    import torch
+    heads, kvh, D, P = 8, 2, 64, 1500
+    calls = []
+    for i in range(12):
+        g = torch.Generator(device=gpu).manual_seed(100 + i)
+        calls.append(dict(q=torch.randn(heads * D, generator=g, device=gpu),
+                          kv=torch.randn(P, 2 * kvh * D, generator=g, device=gpu),
+                          ws=torch.zeros(256, dtype=torch.uint8, device=gpu), stream=torch.cuda.Stream(),
+                          out=torch.empty(heads * D, device=gpu)))
+
+    def run(c, out, stream):
+        fmx.call("fmx_attention_decode", c["q"].data_ptr(), c["kv"].data_ptr(), 2 * kvh * D, kvh * D, heads, kvh, D, P,
+                 0.125, out.data_ptr(), c["ws"].data_ptr(), 256, stream)
+
+    want = []
+    for c in calls:
+        run(c, c["out"], fmx.stream_handle())
+        torch.cuda.synchronize()
+        want.append(c["out"].clone())
+    torch.cuda.synchronize()
+    for _ in range(5):
+        for c in calls:
+            c["out"].zero_()
+        torch.cuda.synchronize()
+        for c in calls:
+            run(c, c["out"], c["stream"].cuda_stream)
+        torch.cuda.synchronize()
+        for c, w in zip(calls, want):
+            assert torch.equal(c["out"], w)

@@ -9,8 +9,8 @@
 // (chain c takes k = c mod 16; chains 0..7 are acc0, 8..15 acc1), an 8-element
 // tail into acc0, lane-wise acc0 + acc1, the 8-lane tree sum, then a scalar
 // FMA tail over the last in_dim mod 8 elements.
-#include "chains.hpp"
 #include "matvec.hpp"
+#include "pair.hpp"
 
 namespace fmx {
 
@@ -52,6 +52,28 @@ __global__ __launch_bounds__(kThreads) void matvec_kernel(
         const float v = T::finish(t[i]);
         if (l == 0 && r0 + i < rows) y[r0 + i] = v;
     }
+}
+
+// Two 8-lane groups per row (pair.hpp), 16 rows per workgroup, x as one LDS
+// tile, the rows' first PF chunks requested before it is staged.
+template <class P, int PF>
+__global__ __launch_bounds__(kThreads) void matvec_pair_kernel(
+    const uint8_t *__restrict__ packed, const float *__restrict__ x, float *__restrict__ y, uint32_t rows,
+    uint32_t blocks, uint32_t chunks, uint64_t scale_bytes) {
+    using T = typename P::T;
+    extern __shared__ __align__(16) float lds[];
+    const uint32_t tid = threadIdx.x, l = tid & 7, hf = (tid >> 3) & 1;
+    const uint32_t r = blockIdx.x * (kThreads / 16) + (tid >> 4);
+    const typename T::Row rw = T::row(packed, scale_bytes, blocks, chunks, r < rows ? r : rows - 1, l);
+    const uint8_t *qp = rw.quants + 8 * hf, *sp = P::scales(rw);
+    XBatch<4> xb;
+    load_batch<T>(xb, x, 0, blocks * T::kBlock, tid, kThreads);
+    PairChunk buf[PF + 1];
+    pair_prime<P, PF>(qp, sp, chunks, buf);
+    T::template stage<4, true>(x, 0, blocks, lds, tid, kThreads, xb);
+    __syncthreads();
+    const float v = P::finish(pair_stream<P, PF>(qp, sp, chunks, P::x_of(lds, blocks, 0, l), l, hf, buf));
+    if ((tid & 15) == 0 && r < rows) y[r] = v;
 }
 
 // F32: 16 lanes per row (4 row slots per wavefront, 16 per workgroup).
@@ -153,6 +175,27 @@ int launch_matvec(const PackedGeometry &g, const void *packed, const float *x, f
     return FMX_OK;
 }
 
+// The pair kernel's twice as many wavefronts with seven chunks each in flight
+// serve the matrices whose rows leave the device short of them. [4096 x 4096]
+// matvec_kernel -> pair: Q4_0 14.2 -> 7.2, Q8_0 18.3 -> 7.2, Q4_K 11.8 -> 8.5
+// us; [4096 x 14336] 44.9 -> 13.5, 58.2 -> 18.6, 34.5 -> 20.9. Past max_rows its
+// 17% more instructions per block cost more: Q4_0 [14336 x 4096] 14.9 -> 11.6
+// but [32000 x 4096] 18.9 -> 19.5; Q8_0 there 30.6 -> 27.2; Q4_K [14336 x 4096]
+// 16.8 -> 19.4. (15 chunks in flight: the same up to 4096 rows, slower above.)
+template <class P, int NR>
+int launch_matvec_quant(uint32_t max_rows, const PackedGeometry &g, const void *packed, const float *x, float *y, hipStream_t s) {
+    using T = typename P::T;
+    const size_t lds = static_cast<size_t>(g.blocks) * T::kLdsFloatsPerBlock * sizeof(float);
+    if (g.rows > max_rows || g.blocks % T::kPerChunk != 0 || lds > kMatvecMaxLds)
+        return launch_matvec<T, NR>(g, packed, x, y, s);
+    auto k = matvec_pair_kernel<P, 7>;
+    if (int rc = allow_lds(reinterpret_cast<const void *>(k), lds)) return rc;
+    hipLaunchKernelGGL(k, dim3(div_up(g.rows, kThreads / 16)), dim3(kThreads), lds, s,
+                       static_cast<const uint8_t *>(packed), x, y, g.rows, g.blocks, g.chunks, g.scale_bytes);
+    FMX_LAUNCH_CHECK();
+    return FMX_OK;
+}
+
 } // namespace
 
 } // namespace fmx
@@ -182,9 +225,9 @@ extern "C" int fmx_matvec(uint32_t type_id, const void *packed, const float *x, 
                                static_cast<const float *>(packed), x, y, out_dim, in_dim);
         FMX_LAUNCH_CHECK();
         return FMX_OK;
-    case FMX_TYPE_Q4_0: return launch_matvec<Q40, 2>(g, packed, x, y, s);
-    case FMX_TYPE_Q8_0: return launch_matvec<Q80, 2>(g, packed, x, y, s);
-    case FMX_TYPE_Q4_K: return launch_matvec<Q4K, 1>(g, packed, x, y, s);
+    case FMX_TYPE_Q4_0: return launch_matvec_quant<PairQ40, 2>(16384, g, packed, x, y, s);
+    case FMX_TYPE_Q8_0: return launch_matvec_quant<PairQ80, 2>(32768, g, packed, x, y, s);
+    case FMX_TYPE_Q4_K: return launch_matvec_quant<PairQ4K, 1>(8192, g, packed, x, y, s);
     case FMX_TYPE_Q6_K: {
         // one lane group per row leaves the device short of wavefronts below
         // 32768 rows: split each row's blocks over 4 (fewer than 8192 rows)

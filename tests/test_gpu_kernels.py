@@ -165,3 +165,18 @@ def test_gemm_quant_errors(gpu):
     assert lib.fmx_gemm_quant(8, w.data_ptr(), x.data_ptr(), y.data_ptr(), 1, 4, 48, None) == 3
     assert lib.fmx_gemm_quant(77, w.data_ptr(), x.data_ptr(), y.data_ptr(), 1, 4, 32, None) == 2
     assert lib.fmx_gemm_quant(8, None, x.data_ptr(), y.data_ptr(), 1, 4, 32, None) == 1
+
+
+@pytest.mark.parametrize("t,rows,cols", [
+    # rows of one chunk, around and between the rings of eight chunks (Q4_0
+    # 256 inputs a chunk, Q8_0 128, Q4_K 256), a part chunk at the end (the
+    # 8-lane kernel), x past 64 KiB of LDS and past 128 KiB
+    (2, 1, 256), (2, 17, 1792), (2, 16, 2048), (2, 15, 2304), (2, 33, 4352), (2, 31, 2080), (2, 4, 16384),
+    (2, 3, 28928),
+    (8, 1, 128), (8, 17, 896), (8, 16, 1024), (8, 15, 1152), (8, 33, 2176), (8, 31, 1056), (8, 4, 17408),
+    (8, 3, 33792),
+    (12, 1, 256), (12, 17, 1792), (12, 16, 2048), (12, 15, 2304), (12, 33, 4352), (12, 4, 16384), (12, 3, 33792),
+    # either side of the rows each type's two-group kernel serves
+    (2, 16384, 256), (2, 16385, 256), (8, 32768, 128), (8, 32769, 128), (12, 8192, 256), (12, 8193, 256)])
+def test_matvec_two_groups_per_row_bitwise(gpu, t, rows, cols):
+    test_matvec_bitwise_vs_oracle(gpu, t, rows, cols)

@@ -673,7 +673,10 @@ __device__ inline float chain_layout_logit(const float *hs, const float *rs, uin
 // reference's h bit for bit.
 template <uint32_t NT>
 __global__ __launch_bounds__(NT) __attribute__((aligned(kHotAlign))) void route_rows_kernel(RouteArgs a, const float *__restrict__ x,
-                                                        float *__restrict__ h_out, float *__restrict__ logits) {
+                                                        float *__restrict__ h_out, float *__restrict__ logits,
+                                                        uint32_t *__restrict__ clear) {
+    // the call's error word, as in rmsnorm_kernel
+    if (clear && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *clear = 0;
     constexpr uint32_t P = 4;
     extern __shared__ __align__(16) float lds[];
     const uint32_t H = a.hidden, E = a.experts, tid = threadIdx.x;
@@ -1080,6 +1083,49 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4 / RJ
     }
 }
 
+// gate_up_kernel on 16 lanes per ffn row, lanes 0-7 the gate row's and 8-15
+// the up row's, for calls with too few rows to fill the device: each wavefront
+// has half the chain to run and the rows' first PF chunks in flight. h is one
+// LDS tile.
+template <class T, int PF>
+__global__ __launch_bounds__(kThreads) void gate_up_split_kernel(
+    ExpertArgs a, const float *__restrict__ h, const float *__restrict__ logits, uint32_t *__restrict__ ids,
+    float *__restrict__ w, float *__restrict__ act, uint32_t *__restrict__ status) {
+    extern __shared__ __align__(16) float lds[];
+    const uint32_t tid = threadIdx.x, l = tid & 7, slot = tid >> 4;
+    const bool is_up = tid & 8;
+    const uint32_t rank = blockIdx.y;
+    const uint32_t blocks = a.gu.blocks;
+    // requested in the order of use, as in gate_up_kernel
+    float lv[4];
+    route_logits_load(a.route, logits ? logits : h, lv);
+    const uint32_t given = logits ? 0u : ids[rank];
+    __builtin_amdgcn_sched_barrier(0);
+    XBatch<4> hb;
+    load_batch<T>(hb, h, 0, blocks * T::kBlock, tid, kThreads);
+    __builtin_amdgcn_sched_barrier(0);
+    const uint32_t e = logits ? expert_of_rank_values(a.route, lv, rank, blockIdx.x == 0 && rank == 0, ids, w, status)
+                              : given;
+    if (e >= a.experts) {
+        if (tid == 0 && blockIdx.x == 0) atomicOr(status, STATUS_BAD_EXPERT);
+        return;
+    }
+    const uint32_t F = a.ffn;
+    const uint32_t j = blockIdx.x * (kThreads / 16) + slot;
+    const uint8_t *gate = static_cast<const uint8_t *>(a.gate[e]), *up = static_cast<const uint8_t *>(a.up[e]);
+    typename T::Row rw[1];
+    rw[0] = T::row(is_up ? up : gate, a.gu.scale_bytes, a.gu.blocks_padded, a.gu.chunks, j < F ? j : F - 1, l);
+    float t[1] = {0.0f};
+    const uint32_t c_end = (blocks + T::kPerChunk - 1) / T::kPerChunk;
+    ChunkStream<T, 1, PF> cs;
+    cs.prime(rw, c_end);
+    T::template stage<4, true>(h, 0, blocks, lds, tid, kThreads, hb);
+    __syncthreads();
+    cs.run(0, c_end, c_end, blocks, 0, blocks, lds, l, t);
+    const float v = T::finish(t[0]), u = row_swap8(v);
+    if ((tid & 15) == 0 && j < F) act[static_cast<uint64_t>(rank) * F + j] = swiglu(v, u);
+}
+
 // Down rows of every routed expert of one token, then the combine in rank
 // order (ffn = 0 + w_0 d_0 + w_1 d_1 ..., engine.cpp:1517, 1770) and the
 // residual (engine.cpp:813-816, 1822). Row slot s handles rank s / jpw, row
@@ -1277,6 +1323,8 @@ __global__ __launch_bounds__(kThreads) void down_q6_k_split_kernel(ExpertArgs a,
 constexpr int kGateUpPF = 1;
 constexpr int kDownPF = 7;
 constexpr int kRJ = 1;
+constexpr int kSplitPF = 7;
+constexpr uint32_t kCus = 256;
 
 // Dynamic LDS of the chain kernels (gate/up: one tile of h; down: one tile
 // of every rank's activations); 0 for the 16-lane kernels.
@@ -1313,8 +1361,25 @@ int launch_timed(K k, dim3 grid, size_t lds, hipStream_t s, const hipEvent_t *ke
 template <class TG>
 int launch_gate_up_q(const ExpertArgs &a, const float *h, const float *logits, uint32_t *ids, float *w, float *act,
                      uint32_t *status, hipStream_t s, const hipEvent_t *kev) {
-    auto gu = gate_up_kernel<TG, kRJ, kGateUpPF>;
     const size_t lds = gate_up_lds(a);
+    // Up to two workgroups of gate_up_split_kernel per CU: its wavefronts run
+    // half the chain of gate_up_kernel's (28 rows per workgroup, so fewer than
+    // two per SIMD there), with more chunks in flight. Layers of (hidden, ffn,
+    // top-k), gate_up_kernel -> split, us per token: (4096, 4096, 2) Q4_0 29.5
+    // -> 26.0, Q8_0 38.6 -> 34.2, Q4_K 47.0 -> 40.3; (2048, 1024, 8) Q4_K 39.1
+    // -> 35.5; past that (2048, 5632, 2) the same, (4096, 14336, 2) 52.7 ->
+    // 57.5. Q4_K, whose chains are the longest, also stays on one
+    // gate_up_kernel workgroup per CU where the split leaves some CUs two:
+    // (2048, 768, 8) 34.9 -> 36.2, against 28.6 -> 28.1 for Q4_0.
+    const uint32_t whole = div_up(a.ffn, kThreads / 64 * 7) * a.top_k, split = div_up(a.ffn, kThreads / 16) * a.top_k;
+    if (split <= 2 * kCus && a.gu_tile >= a.gu.blocks &&
+        !(TG::kType == FMX_TYPE_Q4_K && whole <= kCus && split > kCus)) {
+        auto gu = gate_up_split_kernel<TG, kSplitPF>;
+        if (int rc = allow_lds(reinterpret_cast<const void *>(gu), lds)) return rc;
+        return launch_timed(gu, dim3(div_up(a.ffn, kThreads / 16), a.top_k), lds, s, kev, a, h, logits, ids, w,
+                            act, status);
+    }
+    auto gu = gate_up_kernel<TG, kRJ, kGateUpPF>;
     if (int rc = allow_lds(reinterpret_cast<const void *>(gu), lds)) return rc;
     return launch_timed(gu, dim3(div_up(a.ffn, (kThreads / 64 * 7) * kRJ), a.top_k), lds, s, kev, a, h, logits, ids, w,
                         act, status);
@@ -1467,11 +1532,11 @@ int launch_router_quant(const RouteArgs &a, const float *h, uint32_t tokens, flo
 // beyond (each thread holds 16 elements of the token). A block-type router
 // takes RMSNorm into h (which it then needs) and the router rows after it.
 int launch_route_logits(const RouteArgs &a, const float *x, uint32_t tokens, float *h, float *logits,
-                        hipStream_t s) {
+                        hipStream_t s, uint32_t *clear) {
     if (a.hidden > kMaxHidden || a.hidden % 4 || a.experts == 0) return FMX_ERR_SHAPE_MISMATCH;
     if (a.router_type != FMX_TYPE_F32) {
         if (!h) return FMX_ERR_INVALID_ARGUMENT;
-        if (int rc = launch_rmsnorm(a, x, tokens, h, s)) return rc;
+        if (int rc = launch_rmsnorm(a, x, tokens, h, s, clear)) return rc;
         return launch_router_quant(a, h, tokens, logits, s);
     }
     const size_t lds = route_lds_bytes(a.hidden);
@@ -1480,11 +1545,11 @@ int launch_route_logits(const RouteArgs &a, const float *x, uint32_t tokens, flo
     if (a.hidden <= 16 * 256) {
         auto k = route_rows_kernel<256>;
         if (int rc = allow_lds(reinterpret_cast<const void *>(k), lds)) return rc;
-        hipLaunchKernelGGL(k, grid, dim3(256), lds, s, a, x, h, logits);
+        hipLaunchKernelGGL(k, grid, dim3(256), lds, s, a, x, h, logits, clear);
     } else {
         auto k = route_rows_kernel<1024>;
         if (int rc = allow_lds(reinterpret_cast<const void *>(k), lds)) return rc;
-        hipLaunchKernelGGL(k, grid, dim3(1024), lds, s, a, x, h, logits);
+        hipLaunchKernelGGL(k, grid, dim3(1024), lds, s, a, x, h, logits, clear);
     }
     FMX_LAUNCH_CHECK();
     return FMX_OK;
@@ -1519,19 +1584,12 @@ int launch_route_batched(const RouteArgs &a, const float *x, uint32_t tokens, fl
     return FMX_OK;
 }
 
-__global__ void route_clear_kernel(uint32_t *word) { *word = 0; }
-
 int launch_route(const RouteArgs &a, const float *x, uint32_t tokens, float *h, float *logits,
                  uint32_t *ids, float *weights, uint32_t *status, hipStream_t s, bool clear_status) {
     bool routed = false;
-    const bool batched = h && tokens > 1;
-    if (clear_status && !batched) {
-        hipLaunchKernelGGL(route_clear_kernel, dim3(1), dim3(1), 0, s, status);
-        FMX_LAUNCH_CHECK();
-    }
-    if (int rc = batched ? launch_route_batched(a, x, tokens, h, logits, s, ids, weights, status, &routed,
-                                                clear_status ? status : nullptr)
-                         : launch_route_logits(a, x, tokens, h, logits, s))
+    uint32_t *clear = clear_status ? status : nullptr;
+    if (int rc = h && tokens > 1 ? launch_route_batched(a, x, tokens, h, logits, s, ids, weights, status, &routed, clear)
+                                 : launch_route_logits(a, x, tokens, h, logits, s, clear))
         return rc;
     if (routed) return FMX_OK;
     hipLaunchKernelGGL(route_finish_kernel, dim3(tokens), dim3(64), 0, s, a, logits, ids, weights, status);

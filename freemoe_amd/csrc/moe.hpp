@@ -41,12 +41,12 @@ struct DecodeScratch {
 };
 
 // Router logits of `tokens` rows of x ([tokens x experts]); h (optional)
-// receives the normalised rows.
+// receives the normalised rows. clear (optional): the call's error word,
+// zeroed by the first kernel launched here (none of them sets a bit).
 int launch_route_logits(const RouteArgs &a, const float *x, uint32_t tokens, float *h, float *logits,
-                        hipStream_t s);
+                        hipStream_t s, uint32_t *clear = nullptr);
 // launch_route_logits, then ids / weights ([tokens x top_k]) from the logits.
-// clear_status: zero *status first (by the first routing kernel where that
-// is the batched RMSNorm, else by a kernel of its own).
+// clear_status: *status zeroed first (by the first routing kernel).
 int launch_route(const RouteArgs &a, const float *x, uint32_t tokens, float *h, float *logits,
                  uint32_t *ids, float *weights, uint32_t *status, hipStream_t s, bool clear_status = false);
 int prepare_expert_args(const fmx_moe_layer *L, const RouteArgs &route, ExpertArgs *a);

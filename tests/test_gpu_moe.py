@@ -604,3 +604,34 @@ def test_bucket_rejects_duplicate_ids(gpu):
     fmx.call("fmx_moe_bucket", ids.data_ptr(), 3, 2, 4, off.data_ptr(), tl.data_ptr(), rl.data_ptr(),
              ws.data_ptr(), ws.numel(), fmx.stream_handle())
     assert fmx.lib().fmx_moe_status(ws.data_ptr(), fmx.stream_handle()) == 0
+
+
+@pytest.mark.parametrize("t", [wl.Q4_0, wl.Q8_0, wl.Q4_K])
+@pytest.mark.parametrize("H,F,E,K", [
+    # gate and up on 16 lanes a row: rows of one chunk, of one ring of eight
+    # and past it, ffn past a whole number of 16-row workgroups
+    (256, 256, 4, 1), (2048, 768, 8, 4), (2304, 1024, 6, 3), (4352, 256, 3, 2),
+    # one and two workgroups per CU, and just past them (28 rows a workgroup
+    # of the 8-lane kernel)
+    (256, 4096, 3, 1), (256, 2048, 8, 4), (256, 2304, 8, 4), (256, 4096, 4, 2), (256, 4352, 4, 2),
+    # every rank's activations in one batch of 8192 and past it
+    (512, 1024, 10, 8), (512, 1280, 10, 8), (256, 256, 40, 32)])
+def test_decode_split_gate_up_and_batched_down_staging(gpu, H, F, E, K, t):
+    lw = wl.make_layer(H, F, E, K, t, 61 + H + F)
+    assert check_layer(gpu, lw, wl.inputs(H, 2, 62)) == 0
+
+
+def test_decode_clears_the_error_word(gpu):
+    """A stale error word is zeroed by the call itself, for one and several
+    tokens and for a block-type router (whose RMSNorm is a launch of its own)."""
+    import torch
+    for kw in ({}, {"router_type": wl.Q8_0}):
+        lw = wl.make_layer(256, 512, 4, 2, wl.Q4_0, 71, **kw)
+        dl = DeviceLayer(lw, gpu)
+        for tokens in (1, 3):
+            x = torch.from_numpy(wl.inputs(256, tokens, 72)).to(gpu)
+            dl.decode(x)
+            torch.cuda.synchronize()
+            dl.workspace[:4] = 1
+            dl.decode(x)
+            assert dl.status() == 0

@@ -179,6 +179,19 @@ __device__ __forceinline__ float row_bcast(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x150 + M, 0xF, 0xF, true));
 }
 
+// Each quad of lanes permuted: lane i takes lane (kPerm >> 2 i) & 3's value.
+template <int kPerm>
+__device__ __forceinline__ uint32_t quad_perm_u32(uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), kPerm, 0xF, 0xF, true));
+}
+
+// Lane M's value in every lane of each quad of lanes (DPP quad permutation).
+template <uint32_t M>
+__device__ __forceinline__ float quad_bcast(float v) {
+    static_assert(M < 4, "a lane of the quad");
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), M * 0x55, 0xF, 0xF, true));
+}
+
 // hsum8_lanes' value in lanes 0-3 of each 8-lane group only (the other four
 // hold sums that mix in the neighbouring group), for callers that read lane
 // 0 of each group: the first stage takes lane i + 4 by a rotation of the
@@ -230,6 +243,22 @@ __device__ __forceinline__ uint2 ld8nt(const void *p) {
 
 __device__ __forceinline__ float ldf_nt(const float *p) {
     return __builtin_nontemporal_load((const __attribute__((address_space(1))) float *)(p));
+}
+
+// 16, 8 and 4 bytes at any even address.
+typedef fmx_u32x4 fmx_u32x4_a2 __attribute__((aligned(2)));
+typedef fmx_u32x2 fmx_u32x2_a2 __attribute__((aligned(2)));
+typedef uint32_t fmx_u32_a2 __attribute__((aligned(2)));
+__device__ __forceinline__ uint4 ld16u2(const void *p) {
+    const fmx_u32x4 v = *(const __attribute__((address_space(1))) fmx_u32x4_a2 *)(p);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ uint2 ld8u2(const void *p) {
+    const fmx_u32x2 v = *(const __attribute__((address_space(1))) fmx_u32x2_a2 *)(p);
+    return make_uint2(v.x, v.y);
+}
+__device__ __forceinline__ uint32_t ld4u2(const void *p) {
+    return *(const __attribute__((address_space(1))) fmx_u32_a2 *)(p);
 }
 
 // 6-bit scale/min pair j of a Q4_K super-block (quant.cpp:63-71).

@@ -18,7 +18,8 @@ namespace {
 
 constexpr uint32_t kThreads = 256;              // 4 wavefronts
 constexpr uint32_t kLdsBudgetFloats = 8 * 1024; // 32 KiB of x per tile
-constexpr size_t kMatvecMaxLds = 128 * 1024;     // the Q6_K split kernel's x and dots
+constexpr size_t kMatvecMaxLds = 128 * 1024;     // the Q6_K kernel's x and dots
+constexpr uint32_t kQ6Quads = 131072;
 
 template <class T, int NR>
 __global__ __launch_bounds__(kThreads) void matvec_kernel(
@@ -118,48 +119,41 @@ __global__ __launch_bounds__(kThreads) void matvec_q6_k_kernel(const uint8_t *__
     if (c == 0 && r < rows) y[r] = total;
 }
 
-// Q6_K with few rows: G lane groups per row, group g taking blocks
-// g, g + G, ... (each block's dot is independent); the block dots meet in LDS
-// and one lane adds them in block order from 0, as q6_k_row_chains does.
-// kXs: x staged in LDS first (block b at xs + b * kQ6XStride), so each input
-// is read from memory once per workgroup instead of once per row (worth its
-// LDS at 8 rows per workgroup).
-// LDS: (16 / G) rows x blocks dots, then x.
-__host__ __device__ inline uint32_t q6_split_dots_floats(uint32_t rows, uint32_t blocks) {
-    return (rows * blocks + 3u) & ~3u;
-}
-template <uint32_t G, bool kXs>
-__global__ __launch_bounds__(kThreads) void matvec_q6_k_split_kernel(const uint8_t *__restrict__ w,
-                                                                     const float *__restrict__ x,
-                                                                     float *__restrict__ y, uint32_t rows,
-                                                                     uint32_t blocks) {
+// Q6_K with x in LDS (block b at xs + b * kQ6XStride): a quad of lanes works on
+// one block at a time (Q6Quad), G quads per row, quad g taking blocks g,
+// g + G, ... (each block's dot is independent); the block dots meet in LDS and
+// one lane adds them in block order from 0, as q6_k_row_chains does.
+// LDS: NT / 4 / G rows x blocks dots, then x.
+template <uint32_t NT, uint32_t G>
+__global__ __launch_bounds__(NT) void matvec_q6_k_quad_kernel(const uint8_t *__restrict__ w,
+                                                                    const float *__restrict__ x, float *__restrict__ y,
+                                                                    uint32_t rows, uint32_t blocks) {
     extern __shared__ __align__(16) float q6_lds[];
-    constexpr uint32_t kRows = kThreads / 16 / G;
-    float *dots = q6_lds;
-    const uint32_t tid = threadIdx.x, c = tid & 15, grp = tid >> 4;
-    const float *xr = x;
-    uint32_t xstride = 256;
-    if constexpr (kXs) {
-        float *xs = q6_lds + q6_split_dots_floats(kRows, blocks);
-        const float4 *x4 = reinterpret_cast<const float4 *>(x);
-        for (uint32_t q = tid; q < blocks * 64; q += kThreads)
-            reinterpret_cast<float4 *>(xs + (q >> 6) * kQ6XStride)[q & 63] = x4[q];
-        __syncthreads();
-        xr = xs;
-        xstride = kQ6XStride;
-    }
-    const uint32_t lr = grp / G, part = grp % G;
+    constexpr uint32_t kRows = NT / 4 / G;
+    float *dots = q6_lds, *xs = q6_lds + q6_dots_floats(kRows, blocks);
+    const uint32_t tid = threadIdx.x, i = tid & 3, quad = tid >> 2;
+    const uint32_t lr = quad / G, part = quad % G;
     const uint32_t r = blockIdx.x * kRows + lr;
-    const uint32_t rr = r < rows ? r : rows - 1;
-    q6_k_block_dots(w + static_cast<uint64_t>(rr) * blocks * 210, xr, blocks, part, G, c, dots + lr * blocks,
-                    xstride);
+    const uint8_t *row = w + static_cast<uint64_t>(r < rows ? r : rows - 1) * blocks * 210;
+    Q6Quad first;
+    first.load(row + (part < blocks ? part : 0) * 210, i);
+    q6_stage_x(x, blocks * 256, xs, tid, NT);
     __syncthreads();
-    if (tid < kRows && blockIdx.x * kRows + tid < rows) {
-        const float *d = dots + tid * blocks;
-        float total = 0.0f;
-        for (uint32_t b = 0; b < blocks; ++b) total = total + d[b];
-        y[blockIdx.x * kRows + tid] = total;
-    }
+    q6_quad_block_dots(first, row, xs, blocks, part, G, i, dots + lr * blocks);
+    __syncthreads();
+    if (tid < kRows && blockIdx.x * kRows + tid < rows) y[blockIdx.x * kRows + tid] = q6_sum_dots(dots + tid * blocks, blocks);
+}
+
+template <uint32_t NT, uint32_t G>
+int launch_q6_k_quad(const void *w, const float *x, float *y, uint32_t rows, uint32_t blocks, hipStream_t s) {
+    constexpr uint32_t kRows = NT / 4 / G;
+    const size_t lds = (q6_dots_floats(kRows, blocks) + static_cast<size_t>(blocks) * kQ6XStride) * sizeof(float);
+    auto k = matvec_q6_k_quad_kernel<NT, G>;
+    if (int rc = allow_lds(reinterpret_cast<const void *>(k), lds)) return rc;
+    hipLaunchKernelGGL(k, dim3(div_up(rows, kRows)), dim3(NT), lds, s, static_cast<const uint8_t *>(w), x, y,
+                       rows, blocks);
+    FMX_LAUNCH_CHECK();
+    return FMX_OK;
 }
 
 template <class T, int NR>
@@ -229,23 +223,24 @@ extern "C" int fmx_matvec(uint32_t type_id, const void *packed, const float *x, 
     case FMX_TYPE_Q8_0: return launch_matvec_quant<PairQ80, 2>(32768, g, packed, x, y, s);
     case FMX_TYPE_Q4_K: return launch_matvec_quant<PairQ4K, 1>(8192, g, packed, x, y, s);
     case FMX_TYPE_Q6_K: {
-        // one lane group per row leaves the device short of wavefronts below
-        // 32768 rows: split each row's blocks over 4 (fewer than 8192 rows)
-        // or 2 groups
-        const bool four = out_dim < 8192;
-        const uint32_t rows_per_wg = four ? kThreads / 64 : kThreads / 32;
-        const size_t dots = q6_split_dots_floats(rows_per_wg, g.blocks) * sizeof(float);
-        const size_t with_x = dots + static_cast<size_t>(g.blocks) * kQ6XStride * sizeof(float);
-        if (out_dim < 32768 && g.blocks >= 8 && dots <= 64 * 1024) {
-            auto k = four ? matvec_q6_k_split_kernel<4, false>
-                          : with_x <= kMatvecMaxLds ? matvec_q6_k_split_kernel<2, true>
-                                                    : matvec_q6_k_split_kernel<2, false>;
-            const size_t lds = !four && with_x <= kMatvecMaxLds ? with_x : dots;
-            if (int rc = allow_lds(reinterpret_cast<const void *>(k), lds)) return rc;
-            hipLaunchKernelGGL(k, dim3(div_up(out_dim, rows_per_wg)), dim3(kThreads), lds, s,
-                               static_cast<const uint8_t *>(packed), x, y, out_dim, g.blocks);
-            FMX_LAUNCH_CHECK();
-            return FMX_OK;
+        // quads per row: as many as give every SIMD eight wavefronts. Every
+        // workgroup stages x, and long inputs let few share a CU's LDS: there
+        // a row's many quads come in larger workgroups, where the rows fill
+        // the device with them ([4096 x 14336] 18.9 -> 16.2 us; [8000 x 4096]
+        // 8.4 -> 11.3)
+        const size_t with_x = (q6_dots_floats(64, g.blocks) + static_cast<size_t>(g.blocks) * kQ6XStride) * 4;
+        if (with_x <= kMatvecMaxLds) {
+            const uint32_t want = kQ6Quads / out_dim;
+            const bool wide = g.blocks >= 32 && out_dim >= 4096;
+            if (want >= 16 && g.blocks >= 16)
+                return wide ? launch_q6_k_quad<1024, 16>(packed, x, y, out_dim, g.blocks, s)
+                            : launch_q6_k_quad<256, 16>(packed, x, y, out_dim, g.blocks, s);
+            if (want >= 8 && g.blocks >= 8)
+                return wide ? launch_q6_k_quad<512, 8>(packed, x, y, out_dim, g.blocks, s)
+                            : launch_q6_k_quad<256, 8>(packed, x, y, out_dim, g.blocks, s);
+            if (want >= 4 && g.blocks >= 4) return launch_q6_k_quad<256, 4>(packed, x, y, out_dim, g.blocks, s);
+            if (want >= 2 && g.blocks >= 2) return launch_q6_k_quad<256, 2>(packed, x, y, out_dim, g.blocks, s);
+            return launch_q6_k_quad<256, 1>(packed, x, y, out_dim, g.blocks, s);
         }
         hipLaunchKernelGGL(matvec_q6_k_kernel, dim3(div_up(out_dim, kThreads / 16)), dim3(kThreads), 0, s,
                            static_cast<const uint8_t *>(packed), x, y, out_dim, g.blocks);

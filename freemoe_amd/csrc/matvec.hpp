@@ -155,31 +155,152 @@ __device__ inline float q6_k_row_chains(const uint8_t *__restrict__ row, const f
 // on different banks.
 constexpr uint32_t kQ6XStride = 272;
 
-// Dots of blocks b0, b0 + stride, ... (< blocks) of one Q6_K row on 16
-// consecutive lanes, each as in q6_k_row_chains (chain c over elements
-// 16 m + c, the lanes' chains joined), the next block's share requested
-// before a block's chain runs; lane 0 writes block b's dot to out[b]. Block
-// b's 256 inputs start at x + b * xstride (256 in memory; more where x is
-// staged in LDS with padding between blocks).
-__device__ __forceinline__ void q6_k_block_dots(const uint8_t *__restrict__ row, const float *x, uint32_t blocks,
-                                                uint32_t b0, uint32_t stride, uint32_t c, float *out,
-                                                uint32_t xstride = 256) {
-    Q6Lane q[2];
-    if (b0 < blocks) q[0].load(row + static_cast<uint64_t>(b0) * 210, x + static_cast<uint64_t>(b0) * xstride, c);
+// A quad's share of a raw Q6_K block: lane i of four consecutive lanes owns
+// chains 4 i .. 4 i + 3, whose quants lie side by side, so that the fields of
+// four elements come out of each word at a time (285 VALU instructions for 64
+// elements where a lane per chain takes 118 for 16). The quad loads whole
+// 64-byte runs, 16 or 8 bytes a lane, and transposes their words between its
+// lanes: the dwords a lane owns, loaded one by one, cost more in requests than
+// the 40 instructions do ([32000 x 4096] 29.6 against 24.8 us). x must be in
+// LDS (the quads of a wavefront on one block read the same 64 bytes).
+struct Q6Quad {
+    uint32_t ql[2][4], qh[2][2];
+    uint32_t sc; // scales 4 i .. 4 i + 3
+    uint32_t d;
+    // The words as loaded: ql[n][k] is word k of bytes 16 i .. + 15 of half n's
+    // run, qh[n][k] word k of bytes 8 i .. + 7.
+    __device__ __forceinline__ void load(const uint8_t *__restrict__ blk, uint32_t i) {
+#pragma unroll
+        for (uint32_t n = 0; n < 2; ++n) {
+            const uint4 v = ld16u2(blk + 64 * n + 16 * i);
+            ql[n][0] = v.x;
+            ql[n][1] = v.y;
+            ql[n][2] = v.z;
+            ql[n][3] = v.w;
+            const uint2 h = ld8u2(blk + 128 + 32 * n + 8 * i);
+            qh[n][0] = h.x;
+            qh[n][1] = h.y;
+        }
+        sc = ld4u2(blk + 192 + 4 * i);
+        d = *reinterpret_cast<const uint16_t *>(blk + 208);
+    }
+    // Word i of lane k's loads to lane i's word k (ql, two exchange stages);
+    // qh: group a's word i is lane 2 a + i / 2's word i % 2.
+    __device__ __forceinline__ void transpose(uint32_t i, uint32_t (&tl)[2][4], uint32_t (&th)[2][2]) const {
+        const bool b0 = i & 1, b1 = i & 2;
+#pragma unroll
+        for (uint32_t n = 0; n < 2; ++n) {
+            uint32_t w[4] = {ql[n][0], ql[n][1], ql[n][2], ql[n][3]};
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k += 2) {
+                const uint32_t r = lane_xor_u32<1>(b0 ? w[k] : w[k + 1]);
+                w[k] = b0 ? r : w[k];
+                w[k + 1] = b0 ? w[k + 1] : r;
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < 2; ++k) {
+                const uint32_t r = lane_xor_u32<2>(b1 ? w[k] : w[k + 2]);
+                tl[n][k] = b1 ? r : w[k];
+                tl[n][k + 2] = b1 ? w[k + 2] : r;
+            }
+            // (the permutations outside the selects: every lane must run them)
+            const uint32_t e0 = quad_perm_u32<0x50>(qh[n][0]), o0 = quad_perm_u32<0x50>(qh[n][1]); // lanes 0 0 1 1
+            const uint32_t e1 = quad_perm_u32<0xFA>(qh[n][0]), o1 = quad_perm_u32<0xFA>(qh[n][1]); // lanes 2 2 3 3
+            th[n][0] = b0 ? o0 : e0;
+            th[n][1] = b0 ? o1 : e1;
+        }
+    }
+    static __device__ __forceinline__ float signed_byte(uint32_t w, uint32_t b) {
+        return static_cast<float>(static_cast<int32_t>(w << (24 - 8 * b)) >> 24);
+    }
+    // The lane's four chains over sub-block M: element 16 M + c has quant byte
+    // [M / 8][M % 2 + 2 (qt % 2)] and bit pair qt = (M % 8) / 2 of qh
+    // [M / 8][M % 2] (Q6Lane), (d sc[M]) (q - 32). A byte holding q's six bits
+    // at the top, the highest flipped, is 4 (q - 32); d4[j] is d sc / 4 of
+    // sub-block 4 i + j, exact, handed over as the multiply's DPP operand.
+    template <uint32_t M>
+    static __device__ __forceinline__ void sub_block(const uint32_t (&tl)[2][4], const uint32_t (&qx)[2][2],
+                                                     const float (&d4)[4], const float *xb, uint32_t i,
+                                                     float (&acc)[4]) {
+        constexpr uint32_t n = M >> 3, a = M & 1, qt = (M & 7) >> 1;
+        const uint32_t wl = tl[n][a + 2 * (qt & 1)];
+        const uint32_t v = ((qt >= 2 ? wl >> 2 : wl << 2) & 0x3C3C3C3Cu) | ((qx[n][a] << (6 - 2 * qt)) & 0xC0C0C0C0u);
+        const float4 xv = *reinterpret_cast<const float4 *>(xb + 16 * M + 4 * i);
+        const float x[4] = {xv.x, xv.y, xv.z, xv.w};
+#pragma unroll
+        for (uint32_t b = 0; b < 4; ++b)
+            acc[b] = fma_rn(quad_bcast<(M >> 2)>(d4[M & 3]) * signed_byte(v, b), x[b], acc[b]);
+    }
+    template <uint32_t... M>
+    static __device__ __forceinline__ void sub_blocks(const uint32_t (&tl)[2][4], const uint32_t (&qx)[2][2],
+                                                      const float (&d4)[4], const float *xb, uint32_t i,
+                                                      float (&acc)[4], std::integer_sequence<uint32_t, M...>) {
+        (sub_block<M>(tl, qx, d4, xb, i, acc), ...);
+    }
+    // The block's dot_avx2 (every lane of the quad returns it): chains c and
+    // c + 8 meet in lanes i and i ^ 2, then the tree's t_c + t_c+4 in i ^ 1.
+    __device__ __forceinline__ float dot(const float *xb, uint32_t i) const {
+        const float df = half_bits_to_float(d) * 0.25f;
+        float d4[4], acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        uint32_t tl[2][4], qx[2][2];
+        transpose(i, tl, qx);
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            d4[j] = df * signed_byte(sc, j);
+            qx[j >> 1][j & 1] ^= 0xAAAAAAAAu;
+        }
+        sub_blocks(tl, qx, d4, xb, i, acc, std::make_integer_sequence<uint32_t, 16>());
+        float s[4];
+#pragma unroll
+        for (uint32_t b = 0; b < 4; ++b) {
+            const float t = acc[b] + lane_xor<2>(acc[b]);
+            s[b] = t + lane_xor<1>(t);
+        }
+        return (s[0] + s[1]) + (s[2] + s[3]);
+    }
+};
+
+// Dots of blocks b0, b0 + stride, ... (< blocks) of one Q6_K row on a quad
+// (lane i), each as in q6_k_row_chains; `first` holds block b0's share (a kernel
+// requests it before it stages x). x in LDS at kQ6XStride floats a block; lane
+// 0 writes block b's dot to out[b].
+__device__ __forceinline__ void q6_quad_block_dots(const Q6Quad &first, const uint8_t *__restrict__ row,
+                                                   const float *xs, uint32_t blocks, uint32_t b0, uint32_t stride,
+                                                   uint32_t i, float *out) {
+    Q6Quad q[2];
+    q[0] = first;
     for (uint32_t b = b0; b < blocks; b += 2 * stride) {
 #pragma unroll
         for (uint32_t u = 0; u < 2; ++u) {
             const uint32_t bu = b + u * stride;
             if (bu >= blocks) break;
-            const uint32_t nb = bu + stride;
-            if (nb < blocks)
-                q[u ^ 1].load(row + static_cast<uint64_t>(nb) * 210, x + static_cast<uint64_t>(nb) * xstride, c);
-            const float acc = q[u].chain();
-            const float t = acc + lane_xor<8>(acc);
-            const float dot = hsum8_first(t); // exact in every lane, as above
-            if (c == 0) out[bu] = dot;
+            if (bu + stride < blocks) q[u ^ 1].load(row + static_cast<uint64_t>(bu + stride) * 210, i);
+            const float dot = q[u].dot(xs + bu * kQ6XStride, i);
+            if (i == 0) out[bu] = dot;
         }
     }
+}
+
+// n floats of x (whole blocks) into LDS in that layout. The caller's barrier
+// publishes them.
+__device__ __forceinline__ void q6_stage_x(const float *__restrict__ x, uint32_t n, float *xs, uint32_t tid,
+                                           uint32_t nthreads) {
+    const float4 *x4 = reinterpret_cast<const float4 *>(x);
+#pragma unroll 4
+    for (uint32_t q = tid; q < n / 4; q += nthreads)
+        reinterpret_cast<float4 *>(xs + (q >> 6) * kQ6XStride)[q & 63] = x4[q];
+}
+
+// The block dots of a row added in block order from 0.
+__device__ __forceinline__ float q6_sum_dots(const float *d, uint32_t blocks) {
+    float total = 0.0f;
+#pragma unroll 8
+    for (uint32_t b = 0; b < blocks; ++b) total = total + d[b];
+    return total;
+}
+
+__host__ __device__ inline uint32_t q6_dots_floats(uint32_t rows, uint32_t blocks) {
+    return (rows * blocks + 3u) & ~3u;
 }
 
 // Row dots on 16 lanes by type, for kernels that take F32 or Q6_K rows: the

@@ -1267,45 +1267,80 @@ __global__ __launch_bounds__(kThreads) void down_rows16_kernel(ExpertArgs a, con
     }
 }
 
-// Q6_K down rows with G 16-lane groups per row: group g takes blocks g,
-// g + G, ... (each block's dot is independent), the block dots meet in LDS
-// and one lane per row adds them in block order from 0 (as q6_k_row_chains
-// does), then the combine in rank order and the residual. 16 / G slots,
-// 16 / G / top_k rows of every rank per workgroup. LDS: 16 / G slots x
-// blocks floats.
+// Q6_K gate and up rows on quads of lanes (Q6Quad), G per row, h in LDS; slot
+// 2 s is gate row s, 2 s + 1 the up row, of the workgroup's 32 / G. LDS: 64 / G
+// slots x blocks dots, then h.
 template <uint32_t G>
-__global__ __launch_bounds__(kThreads) void down_q6_k_split_kernel(ExpertArgs a, const float *__restrict__ x,
-                                                                   const float *__restrict__ act,
-                                                                   const uint32_t *__restrict__ ids,
-                                                                   const float *__restrict__ w,
-                                                                   float *__restrict__ out,
-                                                                   uint32_t *__restrict__ status) {
-    extern __shared__ float dots[];
-    constexpr uint32_t kSlots = kThreads / 16 / G;
+__global__ __launch_bounds__(kThreads) void gate_up_q6_k_quad_kernel(ExpertArgs a, const float *__restrict__ h,
+                                                                     const float *__restrict__ logits,
+                                                                     uint32_t *__restrict__ ids,
+                                                                     float *__restrict__ w, float *__restrict__ act,
+                                                                     uint32_t *__restrict__ status) {
+    extern __shared__ __align__(16) float q6_lds[];
+    constexpr uint32_t kSlots = kThreads / 4 / G;
+    const uint32_t tid = threadIdx.x, i = tid & 3, quad = tid >> 2, slot = quad / G, part = quad % G;
+    const uint32_t rank = blockIdx.y, F = a.ffn, blocks = a.hidden / 256;
+    float *dots = q6_lds, *xs = q6_lds + q6_dots_floats(kSlots, blocks);
+    float lv[4];
+    route_logits_load(a.route, logits ? logits : h, lv);
+    const uint32_t given = logits ? 0u : ids[rank];
+    __builtin_amdgcn_sched_barrier(0);
+    q6_stage_x(h, a.hidden, xs, tid, kThreads);
+    const uint32_t e = logits ? expert_of_rank_values(a.route, lv, rank, blockIdx.x == 0 && rank == 0, ids, w, status)
+                              : given;
+    if (e >= a.experts) {
+        if (tid == 0 && blockIdx.x == 0) atomicOr(status, STATUS_BAD_EXPERT);
+        return;
+    }
+    const uint32_t j = blockIdx.x * (kSlots / 2) + (slot >> 1);
+    const uint8_t *m = static_cast<const uint8_t *>(slot & 1 ? a.up[e] : a.gate[e]);
+    const uint8_t *row = m + static_cast<uint64_t>(j < F ? j : F - 1) * blocks * 210;
+    Q6Quad first;
+    first.load(row + (part < blocks ? part : 0) * 210, i);
+    __syncthreads();
+    q6_quad_block_dots(first, row, xs, blocks, part, G, i, dots + slot * blocks);
+    __syncthreads();
+    if (tid < kSlots) {
+        const float v = q6_sum_dots(dots + tid * blocks, blocks), u = lane_xor<1>(v);
+        const uint32_t jo = blockIdx.x * (kSlots / 2) + (tid >> 1);
+        if (!(tid & 1) && jo < F) act[static_cast<uint64_t>(rank) * F + jo] = swiglu(v, u);
+    }
+}
+
+// Q6_K down rows on quads of lanes, G per row, every rank's activations in
+// LDS; NT / 4 / G slots, NT / 4 / G / top_k rows of every rank per workgroup,
+// then the combine in rank order and the residual. LDS: NT / 4 / G slots x
+// blocks dots, then the activations.
+template <uint32_t NT, uint32_t G>
+__global__ __launch_bounds__(NT) void down_q6_k_quad_kernel(ExpertArgs a, const float *__restrict__ x,
+                                                                        const float *__restrict__ act,
+                                                                        const uint32_t *__restrict__ ids,
+                                                                        const float *__restrict__ w,
+                                                                        float *__restrict__ out,
+                                                                        uint32_t *__restrict__ status) {
+    extern __shared__ __align__(16) float q6_lds[];
+    constexpr uint32_t kSlots = NT / 4 / G;
     __shared__ float dres[kSlots];
-    const uint32_t tid = threadIdx.x, c = tid & 15, grp = tid >> 4;
-    const uint32_t slot = grp / G, part = grp % G;
+    const uint32_t tid = threadIdx.x, i = tid & 3, quad = tid >> 2, slot = quad / G, part = quad % G;
     const uint32_t K = a.top_k, H = a.hidden, F = a.ffn, blocks = F / 256;
+    float *dots = q6_lds, *xs = q6_lds + q6_dots_floats(kSlots, blocks);
     const uint32_t jpw = kSlots / K;
     const uint32_t rank = slot / jpw < K ? slot / jpw : K - 1;
     const uint32_t j = blockIdx.x * jpw + slot % jpw;
-    const uint32_t jr = j < H ? j : H - 1;
     uint32_t e = ids[rank];
-    const bool bad = e >= a.experts;
-    if (bad) {
-        if (c == 0 && part == 0) atomicOr(status, STATUS_BAD_EXPERT);
+    if (e >= a.experts) {
+        if (i == 0 && part == 0) atomicOr(status, STATUS_BAD_EXPERT);
         e = 0;
     }
-    q6_k_block_dots(static_cast<const uint8_t *>(a.down[e]) + static_cast<uint64_t>(jr) * blocks * 210,
-                    act + static_cast<uint64_t>(rank) * F, blocks, part, G, c, dots + slot * blocks);
+    const uint8_t *row = static_cast<const uint8_t *>(a.down[e]) + static_cast<uint64_t>(j < H ? j : H - 1) * blocks * 210;
+    Q6Quad first;
+    first.load(row + (part < blocks ? part : 0) * 210, i);
+    q6_stage_x(act, K * F, xs, tid, NT);
     __syncthreads();
-    if (tid < K * jpw) {
-        // slot tid: rank tid / jpw
-        const float *d = dots + tid * blocks;
-        float v = 0.0f;
-        for (uint32_t b = 0; b < blocks; ++b) v = v + d[b];
-        dres[tid] = ids[tid / jpw] >= a.experts ? 0.0f : v;
-    }
+    q6_quad_block_dots(first, row, xs + rank * blocks * kQ6XStride, blocks, part, G, i, dots + slot * blocks);
+    __syncthreads();
+    if (tid < K * jpw) // slot tid: rank tid / jpw
+        dres[tid] = ids[tid / jpw] >= a.experts ? 0.0f : q6_sum_dots(dots + tid * blocks, blocks);
     __syncthreads();
     if (tid < jpw) {
         const uint32_t jo = blockIdx.x * jpw + tid;
@@ -1325,6 +1360,7 @@ constexpr int kDownPF = 7;
 constexpr int kRJ = 1;
 constexpr int kSplitPF = 7;
 constexpr uint32_t kCus = 256;
+constexpr uint32_t kQ6Quads = 65536;
 
 // Dynamic LDS of the chain kernels (gate/up: one tile of h; down: one tile
 // of every rank's activations); 0 for the 16-lane kernels.
@@ -1396,6 +1432,30 @@ int launch_down_q(const ExpertArgs &a, const float *x, const float *act, const u
     return launch_timed(dn, dim3(div_up(a.hidden, jpw)), lds, s, kev, a, x, act, ids, w, out, status);
 }
 
+template <uint32_t G>
+int launch_gate_up_q6_k(const ExpertArgs &a, const float *h, const float *logits, uint32_t *ids, float *w, float *act,
+                        uint32_t *status, hipStream_t s, const hipEvent_t *kev) {
+    constexpr uint32_t kSlots = kThreads / 4 / G;
+    const uint32_t blocks = a.hidden / 256;
+    const size_t lds = (q6_dots_floats(kSlots, blocks) + static_cast<size_t>(blocks) * kQ6XStride) * sizeof(float);
+    auto k = gate_up_q6_k_quad_kernel<G>;
+    if (int rc = allow_lds(reinterpret_cast<const void *>(k), lds)) return rc;
+    return launch_timed(k, dim3(div_up(a.ffn, kSlots / 2), a.top_k), lds, s, kev, a, h, logits, ids, w, act, status);
+}
+
+// Quads per Q6_K gate/up row: two up to eight wavefronts per SIMD, more only up
+// to four, since every workgroup routes and stages h itself (layers of
+// (hidden, ffn, top-k), us per token: (4096, 14336, 2) one quad 88.4, two 81.0;
+// (2048, 768, 8) four 31.0, eight 38.5).
+int launch_gate_up_q6_k(const ExpertArgs &a, const float *h, const float *logits, uint32_t *ids, float *w, float *act,
+                        uint32_t *status, hipStream_t s, const hipEvent_t *kev) {
+    const uint32_t rows = 2 * a.ffn * a.top_k, blocks = a.hidden / 256;
+    if (rows * 8 <= kQ6Quads && blocks >= 8) return launch_gate_up_q6_k<8>(a, h, logits, ids, w, act, status, s, kev);
+    if (rows * 4 <= kQ6Quads && blocks >= 4) return launch_gate_up_q6_k<4>(a, h, logits, ids, w, act, status, s, kev);
+    if (rows <= kQ6Quads && blocks >= 2) return launch_gate_up_q6_k<2>(a, h, logits, ids, w, act, status, s, kev);
+    return launch_gate_up_q6_k<1>(a, h, logits, ids, w, act, status, s, kev);
+}
+
 int launch_gate_up(const ExpertArgs &a, const float *h, const float *logits, uint32_t *ids, float *w, float *act,
                    uint32_t *status, hipStream_t s, const hipEvent_t *kev) {
     const dim3 grid16(div_up(a.ffn, kThreads / 16), a.top_k);
@@ -1404,8 +1464,7 @@ int launch_gate_up(const ExpertArgs &a, const float *h, const float *logits, uin
         return launch_timed(gate_up_rows16_kernel<FMX_TYPE_F32>, grid16, a.hidden * sizeof(float), s, kev, a, h, logits,
                             ids, w, act, status);
     case FMX_TYPE_Q6_K:
-        return launch_timed(gate_up_rows16_kernel<FMX_TYPE_Q6_K>, grid16, a.hidden * sizeof(float), s, kev, a, h, logits,
-                            ids, w, act, status);
+        return launch_gate_up_q6_k(a, h, logits, ids, w, act, status, s, kev);
     case FMX_TYPE_Q4_0: return launch_gate_up_q<Q40>(a, h, logits, ids, w, act, status, s, kev);
     case FMX_TYPE_Q8_0: return launch_gate_up_q<Q80>(a, h, logits, ids, w, act, status, s, kev);
     case FMX_TYPE_Q4_K: return launch_gate_up_q<Q4K>(a, h, logits, ids, w, act, status, s, kev);
@@ -1413,15 +1472,46 @@ int launch_gate_up(const ExpertArgs &a, const float *h, const float *logits, uin
     return FMX_ERR_UNSUPPORTED_QUANTISATION;
 }
 
-// down_q6_k_split_kernel<G>: 16 / G row slots over the ranks per workgroup.
-template <uint32_t G>
-int launch_down_q6_k_split(const ExpertArgs &a, const float *x, const float *act, const uint32_t *ids,
-                           const float *w, float *out, uint32_t *status, hipStream_t s, const hipEvent_t *kev) {
-    constexpr uint32_t kSlots = kThreads / 16 / G;
-    const size_t lds = static_cast<size_t>(kSlots) * (a.ffn / 256) * sizeof(float);
-    if (int rc = allow_lds(reinterpret_cast<const void *>(down_q6_k_split_kernel<G>), lds)) return rc;
-    return launch_timed(down_q6_k_split_kernel<G>, dim3(div_up(a.hidden, kSlots / a.top_k)), lds, s, kev, a, x, act,
-                        ids, w, out, status);
+template <uint32_t NT, uint32_t G>
+int launch_down_q6_k(const ExpertArgs &a, const float *x, const float *act, const uint32_t *ids, const float *w,
+                     float *out, uint32_t *status, size_t lds, hipStream_t s, const hipEvent_t *kev) {
+    auto k = down_q6_k_quad_kernel<NT, G>;
+    if (int rc = allow_lds(reinterpret_cast<const void *>(k), lds)) return rc;
+    const dim3 grid(div_up(a.hidden, NT / 4 / G / a.top_k));
+    if (kev)
+        hipExtLaunchKernelGGL(k, grid, dim3(NT), lds, s, kev[0], kev[1], 0, a, x, act, ids, w, out, status);
+    else
+        hipLaunchKernelGGL(k, grid, dim3(NT), lds, s, a, x, act, ids, w, out, status);
+    FMX_LAUNCH_CHECK();
+    return FMX_OK;
+}
+
+// Q6_K down rows on quads, where every rank's activations fit the LDS
+// (*done: whether they do). A workgroup per CU takes hidden / 256 rows of
+// every rank; its quads, 64 or 256, go to as many blocks of a row at once as
+// there are (at most 16).
+int launch_down_q6_k(const ExpertArgs &a, const float *x, const float *act, const uint32_t *ids, const float *w,
+                     float *out, uint32_t *status, hipStream_t s, const hipEvent_t *kev, bool *done) {
+    const uint32_t slots = div_up(a.hidden, kCus) * a.top_k, blocks = a.ffn / 256;
+    const bool small = slots * (blocks < 16 ? blocks : 16) <= 64;
+    const uint32_t quads = small ? 64 : 256;
+    uint32_t G = 16;
+    while (G > 2 && (G > blocks || G * slots > quads)) G /= 2;
+    const size_t lds =
+        (q6_dots_floats(quads / G, blocks) + static_cast<size_t>(a.top_k) * blocks * kQ6XStride) * sizeof(float);
+    *done = a.top_k <= quads / G && lds <= kMaxLds - 2048;
+    if (!*done) return FMX_OK;
+    auto pick = [&](auto g) {
+        constexpr uint32_t kG = decltype(g)::value;
+        return small ? launch_down_q6_k<256, kG>(a, x, act, ids, w, out, status, lds, s, kev)
+                     : launch_down_q6_k<1024, kG>(a, x, act, ids, w, out, status, lds, s, kev);
+    };
+    switch (G) {
+    case 16: return pick(std::integral_constant<uint32_t, 16>());
+    case 8: return pick(std::integral_constant<uint32_t, 8>());
+    case 4: return pick(std::integral_constant<uint32_t, 4>());
+    default: return pick(std::integral_constant<uint32_t, 2>());
+    }
 }
 
 int launch_down(const ExpertArgs &a, const float *x, const float *act, const uint32_t *ids, const float *w,
@@ -1432,15 +1522,13 @@ int launch_down(const ExpertArgs &a, const float *x, const float *act, const uin
     switch (a.type_dn) {
     case FMX_TYPE_F32:
         return launch_timed(down_rows16_kernel<FMX_TYPE_F32>, grid16(), 0, s, kev, a, x, act, ids, w, out, status);
-    case FMX_TYPE_Q6_K:
-        // Q6_K rows of many blocks split over four (or two) lane groups
-        // each, while every rank keeps a row slot
-        if (a.top_k <= kThreads / 64 && a.ffn / 256 >= 8)
-            return launch_down_q6_k_split<4>(a, x, act, ids, w, out, status, s, kev);
-        if (a.top_k <= kThreads / 32 && a.ffn / 256 >= 8)
-            return launch_down_q6_k_split<2>(a, x, act, ids, w, out, status, s, kev);
+    case FMX_TYPE_Q6_K: {
+        bool done;
+        if (int rc = launch_down_q6_k(a, x, act, ids, w, out, status, s, kev, &done)) return rc;
+        if (done) return FMX_OK;
         return launch_timed(down_rows16_kernel<FMX_TYPE_Q6_K>, grid16(), 0, s, kev, a, x, act, ids, w, out,
                             status);
+    }
     case FMX_TYPE_Q4_0:
         if (pair_down_fits<PairQ40>(a)) return launch_down_pair<PairQ40>(a, x, act, ids, w, out, status, s, kev);
         return launch_down_q<Q40>(a, x, act, ids, w, out, status, s, kev);

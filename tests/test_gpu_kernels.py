@@ -180,3 +180,14 @@ def test_gemm_quant_errors(gpu):
     (2, 16384, 256), (2, 16385, 256), (8, 32768, 128), (8, 32769, 128), (12, 8192, 256), (12, 8193, 256)])
 def test_matvec_two_groups_per_row_bitwise(gpu, t, rows, cols):
     test_matvec_bitwise_vs_oracle(gpu, t, rows, cols)
+
+
+@pytest.mark.parametrize("rows,cols", [
+    # one, two, four, eight and sixteen quads a row, at and past their rows and
+    # block counts, rows past whole workgroups, the large workgroups of long
+    # rows, and inputs past the LDS (16 lanes a row)
+    (131073, 256), (65537, 512), (65536, 512), (40000, 256), (32769, 1024), (32768, 1024), (16385, 2048), (16384, 2048),
+    (16383, 1792), (8193, 4096), (8192, 4096), (8191, 3840), (5, 4096), (1, 256), (3, 768), (4099, 8192), (4095, 8192),
+    (9001, 8192), (7, 29440), (5, 30208), (3, 33792)])
+def test_matvec_q6_k_quads_bitwise(gpu, rows, cols):
+    test_matvec_bitwise_vs_oracle(gpu, 14, rows, cols)

@@ -635,3 +635,14 @@ def test_decode_clears_the_error_word(gpu):
             dl.workspace[:4] = 1
             dl.decode(x)
             assert dl.status() == 0
+
+
+@pytest.mark.parametrize("H,F,E,K", [
+    # Q6_K gate/up on one, two, four and eight quads a row; down on two to
+    # sixteen, in small and large workgroups; rows past whole workgroups;
+    # activations past the LDS (16 lanes a row)
+    (256, 256, 3, 1), (512, 512, 4, 2), (1024, 768, 10, 8), (2048, 1024, 6, 2), (2048, 2304, 4, 2), (256, 8192, 3, 2),
+    (256, 33024, 3, 2), (2304, 256, 6, 4), (1280, 4096, 4, 1), (512, 5120, 18, 16), (512, 2560, 18, 16)])
+def test_decode_q6_k_quads(gpu, H, F, E, K):
+    lw = wl.make_layer(H, F, E, K, wl.Q6_K, 91 + H + F)
+    assert check_layer(gpu, lw, wl.inputs(H, 2, 92)) == 0

@@ -27,12 +27,15 @@
 
 #include <hip/hip_ext.h>
 
+#include <type_traits>
+
 namespace fmx {
 
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -89,6 +92,14 @@ struct GQ80 {
         for (int i = 0; i < 4; ++i) w.q[i] = ld16(q + 16 * i);
         w.d = ld8(packed + static_cast<uint64_t>(r) * g.blocks_padded * 2 + static_cast<uint64_t>(step) * 8);
     }
+    // SmallWave's quarter of a chunk (one step): slices 2 g and 2 g + 1.
+    __device__ static void load_quarter(WStep &w, const uint8_t *packed, const PackedGeometry &g, uint32_t r,
+                                        uint32_t chunk, uint32_t quarter) {
+        const uint8_t *q = packed + g.scale_bytes + (static_cast<uint64_t>(r) * g.chunks + chunk) * 128 + quarter * 32;
+        w.q[0] = ld16(q);
+        w.q[1] = ld16(q + 16);
+        w.d = ld8(packed + static_cast<uint64_t>(r) * g.blocks_padded * 2 + static_cast<uint64_t>(chunk) * 8);
+    }
     // The step's block scales as floats (once per step, not per K slice).
     struct Dec {
         float d[4];
@@ -140,6 +151,14 @@ struct GQ40 {
         w.q[0] = ld16(q);
         w.q[1] = ld16(q + 16);
         w.d = ld16(packed + static_cast<uint64_t>(r) * g.blocks_padded * 2 + static_cast<uint64_t>(c) * 16);
+    }
+    // SmallWave's quarter of a chunk (two steps): slices g and 4 + g.
+    __device__ static void load_quarter(WStep &w, const uint8_t *packed, const PackedGeometry &g, uint32_t r,
+                                        uint32_t chunk, uint32_t quarter) {
+        const uint8_t *q = packed + g.scale_bytes + ((static_cast<uint64_t>(r) * g.chunks + chunk) * 8 + quarter) * 16;
+        w.q[0] = ld16(q);
+        w.q[1] = ld16(q + 64);
+        w.d = ld16(packed + static_cast<uint64_t>(r) * g.blocks_padded * 2 + static_cast<uint64_t>(chunk) * 16);
     }
     // The chunk's block scales as 2^9 d and -8 d, once per step.
     struct Dec {
@@ -201,6 +220,15 @@ struct GQ4K {
         w.q[0] = ld16(q);
         w.q[1] = ld16(q + 16);
         w.hd = ld16(packed + (static_cast<uint64_t>(r) * g.chunks + c) * 16);
+    }
+    // SmallWave's quarter of a chunk (two steps): slices g and 4 + g.
+    __device__ static void load_quarter(WStep &w, const uint8_t *packed, const PackedGeometry &g, uint32_t r,
+                                        uint32_t chunk, uint32_t quarter) {
+        const uint64_t c = static_cast<uint64_t>(r) * g.chunks + chunk;
+        const uint8_t *q = packed + g.scale_bytes + (c * 8 + quarter) * 16;
+        w.q[0] = ld16(q);
+        w.q[1] = ld16(q + 64);
+        w.hd = ld16(packed + c * 16);
     }
     // The super-block's sub-block scales 2^9 d sc_j and negated mins
     // -dmin m_j (j < 8) as floats, once per step; the products are exact in
@@ -671,6 +699,207 @@ __global__ __launch_bounds__(kGThreads) __attribute__((amdgpu_waves_per_eu(2, 2)
     }
 }
 
+// ---------------------------------------------------- the GEMMs, few rows --
+//
+// Row tiles of at most 64 pairs (a call of up to 64 tokens: an expert gets a
+// token at most once) are bound by the weight stream: the tiles above, one
+// lane per weight row, spread each load over 64 runs of 16 bytes, and the
+// per-CU request path, not HBM, set their time (more workgroups per CU or
+// deeper prefetch gave 8%). Here a wavefront takes 16 weight rows of two
+// matrices (gate/up: the same 16 ffn rows of both, so SwiGLU needs no
+// exchange; down: 32 rows), a row's 128-byte chunk on four lanes next to
+// each other, for v_mfma_f32_16x16x32_bf16: A lane l =
+// tile row 16 i + l % 16, B lane l = weight row l % 16, both at positions 32 q
+// + 8 j .. + 8 of the step for q = l / 16 and slice j; C element r of lane l =
+// row 4 q + r, column l % 16. Activations go through three LDS buffers (as
+// above, 16 rows per pass of the workgroup's four wavefronts), weights through
+// three register slots of a chunk (one step of Q8_0, two of Q4_0 and Q4_K),
+// requested two steps and two chunks ahead and left in flight across the
+// steps' barriers.
+// Mixtral-shaped layer, 33 tokens, against the kernels above: Q4_0 gate/up 187
+// -> 140 us (3.8 TB/s), down 89 -> 74, the call 313 -> 250; Q8_0 467 -> 397;
+// Q4_K gate/up 221 -> 174. (Non-temporal weight loads: 260; three wavefronts
+// per SIMD spill; a ring slot per 64 bytes of a row instead of a chunk: 273.)
+constexpr uint32_t kSThreads = 256;
+constexpr uint32_t kSmallRows = 64;
+
+template <class T, uint32_t NB>
+struct SmallWave {
+    typename T::WStep w[3][2];
+    typename T::Dec dc[2];
+    f32x4 acc[2][NB];
+    const __bf16 *xrow[NB];
+    static constexpr uint32_t kPerChunk = T::kChunkK / kGStepK; // steps
+
+    __device__ __forceinline__ void load_x(char *dst, uint32_t k0) {
+#pragma unroll
+        for (uint32_t i = 0; i < NB; ++i) load_lds16(xrow[i] + k0, dst + i * 16 * kGRowBytes);
+    }
+
+    // Step `half` of the chunk in ring slot `slot`.
+    __device__ __forceinline__ void multiply(int slot, uint32_t half, const char *buf, uint32_t lane) {
+        const uint32_t row = lane & 15, q = lane >> 4;
+        if (half == 0) {
+#pragma unroll
+            for (int m = 0; m < 2; ++m) T::decode(w[slot][m], dc[m]);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            bf16x8 av[NB], bv[2];
+            const char *a = buf + row * kGRowBytes + (((4 * q + j) ^ row) << 4);
+#pragma unroll
+            for (uint32_t i = 0; i < NB; ++i)
+                av[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4 *>(a + i * 16 * kGRowBytes));
+#pragma unroll
+            for (int m = 0; m < 2; ++m) bv[m] = T::dequant_kk(w[slot][m], dc[m], 4 * half + j);
+#pragma unroll
+            for (uint32_t i = 0; i < NB; ++i)
+#pragma unroll
+                for (int m = 0; m < 2; ++m)
+                    acc[m][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bv[m], acc[m][i], 0, 0, 0);
+        }
+    }
+
+    // K steps [s0, s0 + steps), s0 at a chunk's start, against weight rows (m0,
+    // r0) and (m1, r1);
+    // staging row r of the tile (r < 16 NB) is row_of(r).
+    template <class RowOf>
+    __device__ __forceinline__ void run(const uint8_t *m0, uint32_t r0, const uint8_t *m1, uint32_t r1,
+                                        const PackedGeometry &g, RowOf row_of, uint32_t s0, uint32_t steps,
+                                        uint32_t buf_bytes, char *lds) {
+        const uint32_t tid = threadIdx.x, lane = tid & 63, quarter = lane >> 4, sr = tid >> 4;
+        const uint32_t wbase = 1024 * __builtin_amdgcn_readfirstlane(tid >> 6);
+        const uint32_t last = s0 + steps - 1;
+        auto clampk = [last](uint32_t k) { return k < last ? k : last; };
+#pragma unroll
+        for (uint32_t i = 0; i < NB; ++i) xrow[i] = row_of(sr + 16 * i) + 8 * ((lane & 15) ^ sr);
+#pragma unroll
+        for (uint32_t i = 0; i < NB; ++i)
+#pragma unroll
+            for (int m = 0; m < 2; ++m) acc[m][i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        const uint32_t c0 = s0 / kPerChunk, c_last = last / kPerChunk;
+        auto request_x = [&](uint32_t buf, uint32_t st) { load_x(lds + buf * buf_bytes + wbase, clampk(st) * kGStepK); };
+        auto request_w = [&](uint32_t slot, uint32_t c) {
+            c = c < c_last ? c : c_last;
+            T::load_quarter(w[slot][0], m0, g, r0, c, quarter);
+            T::load_quarter(w[slot][1], m1, g, r1, c, quarter);
+        };
+        request_x(0, s0);
+        request_w(0, c0);
+        request_x(1, s0 + 1);
+        request_w(1, c0 + 1);
+        wait_vm_lgkm0<0>();
+        __syncthreads();
+        auto step = [&](uint32_t u, uint32_t st) { // u = (st - s0) % 6
+            request_x((u + 2) % 3, st + 2);        // the buffer step st - 1 read
+            __builtin_amdgcn_sched_barrier(0);
+            if (u % kPerChunk == 0) request_w((u / kPerChunk + 2) % 3, st / kPerChunk + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(u / kPerChunk % 3, u % kPerChunk, lds + u % 3 * buf_bytes, lane);
+            __builtin_amdgcn_sched_barrier(0);
+            // step st + 1's activations: older than this step's and than the
+            // four quant loads of the newest chunk
+            wait_vm_lgkm0<NB + 4>();
+            lds_barrier();
+        };
+        constexpr uint32_t kPass = 6; // one basic block: its first step waits for every load
+        uint32_t s = 0;
+        for (; s + kPass <= steps; s += kPass) {
+#pragma unroll
+            for (uint32_t u = 0; u < kPass; ++u) step(u, s0 + s + u);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kPass; ++u) {
+            if (s + u >= steps) break;
+            step(u, s0 + s + u);
+        }
+        wait_vm_lgkm0<0>(); // no direct-to-LDS load outlives the workgroup
+    }
+};
+
+template <class T, uint32_t NB>
+__device__ __forceinline__ void small_gate_up_tile(const ExpertArgs &a, uint32_t e, uint32_t row0, uint32_t rows,
+                                                   uint32_t pairs, uint32_t tokens, const __bf16 *__restrict__ hb,
+                                                   const uint32_t *__restrict__ token_list, __bf16 *__restrict__ act,
+                                                   uint32_t buf_bytes, char *lds) {
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t f = blockIdx.x * 64 + 16 * wave + (lane & 15), H = a.hidden, F = a.ffn;
+    auto row_of = [=](uint32_t r) { // as in gate_up_tile
+        const uint32_t pr = row0 + r < pairs ? row0 + r : pairs - 1, t = token_list[pr];
+        return hb + static_cast<uint64_t>(t < tokens ? t : 0u) * H;
+    };
+    SmallWave<T, NB> sw;
+    sw.run(static_cast<const uint8_t *>(a.gate[e]), f, static_cast<const uint8_t *>(a.up[e]), f, a.gu, row_of, 0,
+           H / kGStepK, buf_bytes, lds);
+    const uint32_t col = down_k_position(a.type_dn, f);
+#pragma unroll
+    for (uint32_t i = 0; i < NB; ++i)
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+            const uint32_t m = 16 * i + 4 * (lane >> 4) + r;
+            if (m >= rows) continue;
+            const float gv = sw.acc[0][i][r], uv = sw.acc[1][i][r];
+            act[static_cast<uint64_t>(row0 + m) * F + col] = static_cast<__bf16>(gv / (1.0f + expf(-gv)) * uv);
+        }
+}
+
+template <class T, uint32_t NB>
+__device__ __forceinline__ void small_down_tile(const ExpertArgs &a, uint32_t e, uint32_t row0, uint32_t rows,
+                                                uint32_t pairs, const __bf16 *__restrict__ act, uint32_t steps,
+                                                float *__restrict__ dn, uint32_t buf_bytes, char *lds) {
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t n = blockIdx.x * 128 + 32 * wave + (lane & 15), H = a.hidden, F = a.ffn;
+    const uint8_t *wd = static_cast<const uint8_t *>(a.down[e]);
+    auto row_of = [=](uint32_t r) { return act + static_cast<uint64_t>(row0 + r) * F; };
+    SmallWave<T, NB> sw;
+    sw.run(wd, n, wd, n + 16, a.dn, row_of, blockIdx.y * steps, steps, buf_bytes, lds);
+    float *dst = dn + static_cast<uint64_t>(blockIdx.y) * pairs * H;
+#pragma unroll
+    for (uint32_t i = 0; i < NB; ++i)
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r) {
+            const uint32_t m = 16 * i + 4 * (lane >> 4) + r;
+            if (m >= rows) continue;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) dst[static_cast<uint64_t>(row0 + m) * H + n + 16 * c] = sw.acc[c][i][r];
+        }
+}
+
+// grid: (ffn / 64, max row tiles).
+template <class T>
+__global__ __launch_bounds__(kSThreads) __attribute__((amdgpu_waves_per_eu(2))) void small_gate_up_kernel(
+    ExpertArgs a, const uint32_t *__restrict__ tiles, const uint32_t *__restrict__ order, uint32_t pairs,
+    uint32_t tokens, const __bf16 *__restrict__ hb, const uint32_t *__restrict__ token_list, __bf16 *__restrict__ act,
+    uint32_t buf_bytes) {
+    extern __shared__ __align__(16) char xlds[];
+    uint32_t e, row0, rows;
+    if (blockIdx.y >= tiles[0] || !row_tile(tiles, order[blockIdx.y], a.experts, pairs, e, row0, rows) ||
+        rows * kGRowBytes > buf_bytes)
+        return;
+    switch ((rows + 15) / 16) {
+    case 1: small_gate_up_tile<T, 1>(a, e, row0, rows, pairs, tokens, hb, token_list, act, buf_bytes, xlds); break;
+    case 2: small_gate_up_tile<T, 2>(a, e, row0, rows, pairs, tokens, hb, token_list, act, buf_bytes, xlds); break;
+    case 3: small_gate_up_tile<T, 3>(a, e, row0, rows, pairs, tokens, hb, token_list, act, buf_bytes, xlds); break;
+    default: small_gate_up_tile<T, 4>(a, e, row0, rows, pairs, tokens, hb, token_list, act, buf_bytes, xlds); break;
+    }
+}
+
+// grid: (hidden / 128, K splits, max row tiles).
+template <class T>
+__global__ __launch_bounds__(kSThreads) __attribute__((amdgpu_waves_per_eu(2))) void small_down_kernel(
+    ExpertArgs a, const uint32_t *__restrict__ tiles, uint32_t pairs, const __bf16 *__restrict__ act, uint32_t steps,
+    float *__restrict__ dn, uint32_t buf_bytes) {
+    extern __shared__ __align__(16) char xlds[];
+    uint32_t e, row0, rows;
+    if (!row_tile(tiles, blockIdx.z, a.experts, pairs, e, row0, rows) || rows * kGRowBytes > buf_bytes) return;
+    switch ((rows + 15) / 16) {
+    case 1: small_down_tile<T, 1>(a, e, row0, rows, pairs, act, steps, dn, buf_bytes, xlds); break;
+    case 2: small_down_tile<T, 2>(a, e, row0, rows, pairs, act, steps, dn, buf_bytes, xlds); break;
+    case 3: small_down_tile<T, 3>(a, e, row0, rows, pairs, act, steps, dn, buf_bytes, xlds); break;
+    default: small_down_tile<T, 4>(a, e, row0, rows, pairs, act, steps, dn, buf_bytes, xlds); break;
+    }
+}
+
 // out[t] = x[t] + ((0 + w_0 D_0) + w_1 D_1 ...) in rank order (engine.cpp:1517,
 // 1770, 813-816), each D the sum of the K splits' partial products in split
 // order. V consecutive elements per thread (hidden % V == 0, x and out
@@ -710,33 +939,51 @@ int launch_pack_h(const float *h, uint32_t hidden, uint32_t tokens, __bf16 *hb, 
     return FMX_OK;
 }
 
-template <class T, class TD>
-int launch_gemms(const ExpertArgs &a, const PrefillBuffers &b, uint32_t max_tiles, hipStream_t s, hipEvent_t *kev) {
-    const size_t lds = 2ull * kGBufBytes; // two activation buffers
-    auto gu = gate_up_gemm_kernel<T>;
-    auto dn = down_gemm_kernel<TD>;
-    if (int rc = allow_lds(reinterpret_cast<const void *>(gu), lds)) return rc;
-    if (int rc = allow_lds(reinterpret_cast<const void *>(dn), lds)) return rc;
-    if (b.pairs == 0) return FMX_OK;
-    if (int rc = launch_pack_h<T>(b.h, a.hidden, b.tokens, b.x, s)) return rc;
-    const dim3 gu_grid(a.ffn / 128, max_tiles), dn_grid(a.hidden / 256, b.splits, max_tiles);
-    const uint32_t steps = a.ffn / kGStepK / b.splits;
-    if (kev) {
-        // the launches record kev[0..1] / kev[2..3] at kernel start and end
-        hipExtLaunchKernelGGL(gu, gu_grid, dim3(kGThreads), lds, s, kev[0], kev[1], 0, a, b.tiles, b.tile_order,
-                              b.pairs, b.tokens, b.x, b.token_list, b.act);
-        FMX_LAUNCH_CHECK();
-        hipExtLaunchKernelGGL(dn, dn_grid, dim3(kGThreads), lds, s, kev[2], kev[3], 0, a, b.tiles, b.pairs, b.act,
-                              steps, b.dn);
-        FMX_LAUNCH_CHECK();
-        return FMX_OK;
-    }
-    hipLaunchKernelGGL(gu, gu_grid, dim3(kGThreads), lds, s, a, b.tiles, b.tile_order, b.pairs, b.tokens, b.x,
-                       b.token_list, b.act);
-    FMX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(dn, dn_grid, dim3(kGThreads), lds, s, a, b.tiles, b.pairs, b.act, steps, b.dn);
+template <class K, class... Args>
+int launch_gemm(K k, dim3 grid, uint32_t threads, size_t lds, hipStream_t s, hipEvent_t *kev, Args... args) {
+    if (int rc = allow_lds(reinterpret_cast<const void *>(k), lds)) return rc;
+    if (kev) // the launch records kev[0..1] at kernel start and end
+        hipExtLaunchKernelGGL(k, grid, dim3(threads), lds, s, kev[0], kev[1], 0, args...);
+    else
+        hipLaunchKernelGGL(k, grid, dim3(threads), lds, s, args...);
     FMX_LAUNCH_CHECK();
     return FMX_OK;
+}
+
+// Whether a GEMM of block type T takes the few-row kernels: a token's experts
+// are distinct, so up to 64 tokens no tile has more rows (Q6_K's raw blocks
+// have no 64-byte runs of a row's K step to put on four lanes).
+template <class T>
+bool few_rows(const PrefillBuffers &b) {
+    return !std::is_same_v<T, GQ6K> && b.tokens <= kSmallRows;
+}
+
+template <class T, class TD>
+int launch_gemms(const ExpertArgs &a, const PrefillBuffers &b, uint32_t max_tiles, hipStream_t s, hipEvent_t *kev) {
+    if (b.pairs == 0) return FMX_OK;
+    if (int rc = launch_pack_h<T>(b.h, a.hidden, b.tokens, b.x, s)) return rc;
+    const size_t lds = 2ull * kGBufBytes; // two activation buffers
+    const uint32_t small_buf = div_up(b.tokens, 16) * 16 * kGRowBytes;
+    const uint32_t steps = a.ffn / kGStepK / b.splits;
+    if (few_rows<T>(b)) {
+        if constexpr (!std::is_same_v<T, GQ6K>)
+            if (int rc = launch_gemm(small_gate_up_kernel<T>, dim3(a.ffn / 64, max_tiles), kSThreads, 3 * small_buf, s,
+                                     kev, a, b.tiles, b.tile_order, b.pairs, b.tokens, b.x, b.token_list, b.act,
+                                     small_buf))
+                return rc;
+    } else if (int rc = launch_gemm(gate_up_gemm_kernel<T>, dim3(a.ffn / 128, max_tiles), kGThreads, lds, s, kev, a,
+                                    b.tiles, b.tile_order, b.pairs, b.tokens, b.x, b.token_list, b.act)) {
+        return rc;
+    }
+    hipEvent_t *dev = kev ? kev + 2 : nullptr;
+    // (the K splits start at whole chunks there)
+    if (few_rows<TD>(b) && (b.splits == 1 || steps % 2 == 0)) {
+        if constexpr (!std::is_same_v<TD, GQ6K>)
+            return launch_gemm(small_down_kernel<TD>, dim3(a.hidden / 128, b.splits, max_tiles), kSThreads,
+                               3 * small_buf, s, dev, a, b.tiles, b.pairs, b.act, steps, b.dn, small_buf);
+    }
+    return launch_gemm(down_gemm_kernel<TD>, dim3(a.hidden / 256, b.splits, max_tiles), kGThreads, lds, s, dev, a,
+                       b.tiles, b.pairs, b.act, steps, b.dn);
 }
 
 template <class T>

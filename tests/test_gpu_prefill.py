@@ -173,3 +173,17 @@ def test_prefill_timed_matches_prefill(gpu):
     f32 = DeviceLayer(wl.make_layer(64, 128, 4, 2, wl.F32, 5), gpu)
     with pytest.raises(fmx.FmxError):
         f32.prefill(torch.from_numpy(wl.inputs(64, 4, 6)).to(gpu), kernel_ms=[])
+
+
+@pytest.mark.parametrize("gate_type,down_type", [(wl.Q8_0, wl.Q8_0), (wl.Q4_0, wl.Q4_0), (wl.Q4_K, wl.Q4_K),
+                                                 (wl.Q6_K, wl.Q4_0), (wl.Q8_0, wl.Q6_K)])
+@pytest.mark.parametrize("H,F,E,K,T", [
+    # the few-row GEMMs: one to four 16-row blocks a tile and their edges, K
+    # steps of one pass of six and past it, an odd number of steps per K split
+    # (ffn 768 on few experts), the last call they take and the first they
+    # do not
+    (256, 256, 4, 2, 2), (256, 768, 4, 2, 16), (768, 1024, 3, 3, 17), (2048, 512, 4, 2, 33), (512, 2304, 20, 6, 48),
+    (256, 512, 2, 2, 49), (512, 768, 24, 4, 64), (256, 256, 1, 1, 64), (256, 512, 2, 2, 65)])
+def test_prefill_few_rows(gpu, H, F, E, K, T, gate_type, down_type):
+    lw = wl.make_layer(H, F, E, K, gate_type, 500 + T, down_type=down_type)
+    check_prefill(gpu, lw, wl.inputs(H, T, 501))

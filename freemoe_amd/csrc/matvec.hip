@@ -4,7 +4,7 @@
 // reference's dedicated AVX2 row dots); Q6_K rows, which the reference runs
 // through row_dot_fused_scalar (kernels.cpp:574-590: each block decoded,
 // dotted by dot_avx2, the block's dot added to the row total), use that order
-// on 16 lanes per row; F32 rows use the
+// on quads of lanes, a block each; F32 rows use the
 // reference's gemv_avx2_row order (kernels.cpp:147-167): per row 16 chains
 // (chain c takes k = c mod 16; chains 0..7 are acc0, 8..15 acc1), an 8-element
 // tail into acc0, lane-wise acc0 + acc1, the 8-lane tree sum, then a scalar

@@ -181,3 +181,32 @@ def test_attention_decode_calls_in_flight_share_no_scores(gpu):
         torch.cuda.synchronize()
         for c, w in zip(calls, want):
             assert torch.equal(c["out"], w)
+
+
+def test_attention_decode_captured_and_replayed(gpu):
+    """A captured call, replayed between eager ones: its ticket names one score
+    buffer for every replay, and each replay gives the eager call's bits."""
+    import torch
+    heads, kvh, D, P = 8, 2, 64, 1500
+    g = torch.Generator(device=gpu).manual_seed(9)
+    q = torch.randn(heads * D, generator=g, device=gpu)
+    kv = torch.randn(P, 2 * kvh * D, generator=g, device=gpu)
+    ws = torch.zeros(256, dtype=torch.uint8, device=gpu)
+    out, eager = torch.empty(heads * D, device=gpu), torch.empty(heads * D, device=gpu)
+
+    def run(o):
+        fmx.call("fmx_attention_decode", q.data_ptr(), kv.data_ptr(), 2 * kvh * D, kvh * D, heads, kvh, D, P, 0.125,
+                 o.data_ptr(), ws.data_ptr(), 256, fmx.stream_handle())
+
+    run(out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run(out)
+    for i in range(12):
+        q.normal_(generator=g)
+        run(eager)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), f"replay {i}"

@@ -646,3 +646,11 @@ def test_decode_clears_the_error_word(gpu):
 def test_decode_q6_k_quads(gpu, H, F, E, K):
     lw = wl.make_layer(H, F, E, K, wl.Q6_K, 91 + H + F)
     assert check_layer(gpu, lw, wl.inputs(H, 2, 92)) == 0
+
+
+@pytest.mark.parametrize("H", [4064, 4128, 6176, 16384])
+def test_rmsnorm_sum_interval_ragged_hidden(gpu, H):
+    """The bounded ordered sum between the certificate and the replay, where a
+    thread's consecutive terms end inside a whole number of them: many tokens,
+    so that some fail the first certificate."""
+    test_rmsnorm_in_order_replay_many_tokens(gpu, "normal", H)

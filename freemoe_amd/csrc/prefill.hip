@@ -790,28 +790,33 @@ struct SmallWave {
         request_w(1, c0 + 1);
         wait_vm_lgkm0<0>();
         __syncthreads();
-        auto step = [&](uint32_t u, uint32_t st) { // u = (st - s0) % 6
-            request_x((u + 2) % 3, st + 2);        // the buffer step st - 1 read
+        auto step = [&](auto vm, uint32_t u, uint32_t st) { // u = (st - s0) % 6
+            request_x((u + 2) % 3, st + 2);                 // the buffer step st - 1 read
             __builtin_amdgcn_sched_barrier(0);
             if (u % kPerChunk == 0) request_w((u / kPerChunk + 2) % 3, st / kPerChunk + 2);
             __builtin_amdgcn_sched_barrier(0);
             multiply(u / kPerChunk % 3, u % kPerChunk, lds + u % 3 * buf_bytes, lane);
             __builtin_amdgcn_sched_barrier(0);
-            // step st + 1's activations: older than this step's and than the
-            // four quant loads of the newest chunk
-            wait_vm_lgkm0<NB + 4>();
+            // step st + 1's activations, requested before everything below
+            wait_vm_lgkm0<decltype(vm)::value>();
             lds_barrier();
         };
+        // Newer than they are: this step's activations and, while a later
+        // chunk uses them, the six loads of the newest chunk, of which four
+        // are left in flight. The last steps count the activations alone: the
+        // weight loads there that no step uses are not in the code.
+        const std::integral_constant<uint32_t, NB + 4> with_weights{};
+        const std::integral_constant<uint32_t, NB> alone{};
         constexpr uint32_t kPass = 6; // one basic block: its first step waits for every load
         uint32_t s = 0;
         for (; s + kPass <= steps; s += kPass) {
 #pragma unroll
-            for (uint32_t u = 0; u < kPass; ++u) step(u, s0 + s + u);
+            for (uint32_t u = 0; u < kPass; ++u) step(with_weights, u, s0 + s + u);
         }
 #pragma unroll
         for (uint32_t u = 0; u < kPass; ++u) {
             if (s + u >= steps) break;
-            step(u, s0 + s + u);
+            step(alone, u, s0 + s + u);
         }
         wait_vm_lgkm0<0>(); // no direct-to-LDS load outlives the workgroup
     }

@@ -20,11 +20,11 @@
 // the sum in position order can lie from the parallel one. A probability or
 // an output whose float is the same over that whole interval is the engine's;
 // where one is not, one lane adds the terms in order. For 32 heads of 128 over
-// 8 kv heads and 2000 positions (16 MB of cache: 3 us of HBM) a call takes 20
-// us, three dependent launches of 1, 5 and 11 us, each a chain of memory,
-// LDS and double-precision latencies; walking every sum in order on one
-// workgroup per head took 215 us (32 of the 256 CUs in use). 8192 positions:
-// 50-67 us.
+// 8 kv heads and 2000 positions (16 MB of cache: 3 us of HBM) a call takes 19
+// us, three dependent launches (traced one by one: 1, 5-6 and 12-13 us), each a
+// chain of memory, LDS and double-precision latencies; walking every sum in
+// order on one workgroup per head took 215 us (32 of the 256 CUs in use). 8192
+// positions: 46 us, 83 over 32 kv heads.
 #include <atomic>
 
 #include "fmx_internal.hpp"
@@ -47,32 +47,28 @@ constexpr uint32_t kGroupPad = 4;   // its LDS rows of group sums: the four colu
 // no faster).
 constexpr uint32_t kSplitPositions = 256;
 
-// Scores between the two kernels of a call: slots of device memory, taken and
-// given back on the device. A call's ticket names its slot; the slot is the
-// call's where attention_begin_kernel found it free, until the call's last
-// value workgroup frees it. A call that found its slot taken (more than kSlots
+// Scores between the two kernels of a call: kSlots buffers of device memory,
+// taken in turn. Nothing holds a buffer: a score carries its call's ticket, and
+// a value workgroup that finds another's among its head's (more than kSlots
 // calls in flight, or a replayed graph's fixed ticket meeting another call's)
-// computes the scores in the value kernel. (Taking it in every score
-// workgroup instead saves that launch, 2 us, but its atomics on one address
-// cost 10 ns each: the score kernel 5.8 -> 15.7 us for 504 workgroups.)
-constexpr uint32_t kSlots = 8;
-constexpr uint32_t kSlotFloats = 512 * 1024;
-__device__ __align__(256) float slot_scores[kSlots][kSlotFloats];
-struct Slot {
-    uint32_t owner; // ticket, 0: free
-    uint32_t done;  // value workgroups past their reads
-    uint32_t pad[62];
-};
-__device__ Slot slots[kSlots];
+// computes them all itself. So a call never reads another's scores, whatever
+// runs beside it; executions of one captured call share a ticket, and with it
+// the inputs the scores come from. (Four buffers: as many calls as a process
+// has hardware queues run at once.)
+constexpr uint32_t kSlots = 4;
+constexpr uint32_t kSlotScores = 512 * 1024;
+__device__ __align__(256) uint64_t slot_scores[kSlots][kSlotScores];
 
-__device__ __forceinline__ bool owns_slot(uint32_t ticket) {
-    return ticket != 0 && slots[ticket % kSlots].owner == ticket;
+// One access each, so that a score and its ticket stay together.
+__device__ __forceinline__ void put_score(uint64_t *at, float score, uint32_t ticket) {
+    __hip_atomic_store(at, static_cast<uint64_t>(ticket) << 32 | __builtin_bit_cast(uint32_t, score), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t get_score(const uint64_t *at) {
+    return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ void attention_begin_kernel(uint32_t *status, uint32_t ticket) {
-    *status = 0;
-    if (ticket != 0 && atomicCAS(&slots[ticket % kSlots].owner, 0u, ticket) == 0u) slots[ticket % kSlots].done = 0;
-}
+__global__ void attention_clear_kernel(uint32_t *status) { *status = 0; }
 
 // The dot of one key with one query (doubles in LDS), in index order. fma:
 // the product is exact, so it rounds once, as the engine's multiply and add.
@@ -91,16 +87,15 @@ __device__ __forceinline__ double dot_in_order(const float *k, const double *q, 
     return dot;
 }
 
-// Scores of 32 positions for every query head of one kv head, into the call's
-// slot. The keys are read once, whole rows at a time, into LDS (rows 4 floats
-// apart in banks); a lane runs one (position, head) chain of head_dim fmas.
+// Scores of 32 positions for every query head of one kv head, into the
+// ticket's slot. The keys are read once, whole rows at a time, into LDS (rows 4
+// floats apart in banks); a lane runs one (position, head) chain of head_dim
+// fmas.
 // grid: position tiles x kv heads; LDS: keys, then 4 heads' queries.
 __global__ __launch_bounds__(kScorePos *kScoreHeads) void attention_scores_kernel(
     const float *__restrict__ q, const float *__restrict__ kv, uint64_t row_stride, uint32_t group,
     uint32_t head_dim, uint32_t positions, double scale, uint32_t ticket) {
     extern __shared__ __align__(16) char lds[];
-    __shared__ bool own_s;
-    if (threadIdx.x == 0) own_s = owns_slot(ticket);
     const uint32_t tid = threadIdx.x, kvh = blockIdx.y, t0 = blockIdx.x * kScorePos;
     const uint32_t kstride = head_dim + 4, qstride = head_dim + 2, D4 = head_dim / 4;
     float *ks = reinterpret_cast<float *>(lds);
@@ -114,7 +109,7 @@ __global__ __launch_bounds__(kScorePos *kScoreHeads) void attention_scores_kerne
             *reinterpret_cast<const float4 *>(keys + t * row_stride + 4 * j);
     }
     const uint32_t pos = tid % kScorePos, hs = tid / kScorePos;
-    float *dst = slot_scores[ticket % kSlots] + t0 + pos;
+    uint64_t *dst = slot_scores[ticket % kSlots] + t0 + pos;
     for (uint32_t h0 = 0; h0 < group; h0 += kScoreHeads) {
         const uint32_t nh = group - h0 < kScoreHeads ? group - h0 : kScoreHeads;
         const uint64_t head0 = static_cast<uint64_t>(kvh) * group + h0;
@@ -122,10 +117,9 @@ __global__ __launch_bounds__(kScorePos *kScoreHeads) void attention_scores_kerne
         for (uint32_t i = tid; i < nh * head_dim; i += kScorePos * kScoreHeads)
             qs[i / head_dim * qstride + i % head_dim] = static_cast<double>(q[head0 * head_dim + i]);
         __syncthreads();
-        if (!own_s) return;
         if (hs < nh && t0 + pos < positions)
-            dst[(head0 + hs) * positions] =
-                static_cast<float>(dot_in_order(ks + pos * kstride, qs + hs * qstride, head_dim) * scale);
+            put_score(dst + (head0 + hs) * positions,
+                      static_cast<float>(dot_in_order(ks + pos * kstride, qs + hs * qstride, head_dim) * scale), ticket);
     }
 }
 
@@ -172,13 +166,14 @@ __global__ __launch_bounds__(NT) void attention_values_kernel(
     const float *__restrict__ q, const float *__restrict__ kv, uint64_t row_stride, uint32_t v_offset,
     uint32_t heads, uint32_t group, uint32_t head_dim, uint32_t positions, double scale, float *__restrict__ out,
     uint32_t *__restrict__ status, uint32_t ticket) {
-    constexpr uint32_t kWaves = NT / 64, kGroups = NT / (kSliceDims / 4), kPrefetch = 8;
+    constexpr uint32_t kWaves = NT / 64, kGroups = NT / (kSliceDims / 4);
+    constexpr uint32_t kPrefetch = kTerms > 2 ? 4 : 8; // (8 beside eight terms spill)
     constexpr uint32_t kGroupStride = kGroups + kGroupPad;
     extern __shared__ __align__(16) char lds[];
     __shared__ __align__(16) double qs[kMaxHeadDim];
     __shared__ float red_max[kWaves];
     __shared__ double red_sum[kWaves], red[3][kWaves], err_s[kSliceDims];
-    __shared__ bool own_s;
+    __shared__ bool stale_s[kWaves];
     __shared__ uint32_t flags_s, todo_s; // 1: non-finite score, 2: a probability undecided
     __shared__ double sum_s;
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -193,7 +188,14 @@ __global__ __launch_bounds__(NT) void attention_values_kernel(
     double *gsum = reinterpret_cast<double *>(lds + ((static_cast<size_t>(P) * 8 + 15) & ~static_cast<size_t>(15)));
     float *gabs = reinterpret_cast<float *>(gsum + kSliceDims * kGroupStride);
 
-    // the first positions of this thread's values, in flight during the softmax
+    // the head's scores, then the first positions of this thread's values, which
+    // stay in flight during the softmax
+    uint64_t raw[kTerms];
+    if (ticket != 0) {
+        const uint64_t *src = slot_scores[ticket % kSlots] + static_cast<uint64_t>(head) * P;
+#pragma unroll
+        for (uint32_t i = 0; i < kTerms; ++i) raw[i] = get_score(src + (i * NT + tid < P ? i * NT + tid : P - 1));
+    }
     const uint32_t col = slice * kSliceDims + (tid & 3) * 4, grp = tid >> 2;
     const uint32_t per_group = div_up(P, kGroups);
     const uint32_t v0 = grp * per_group < P ? grp * per_group : P;
@@ -210,18 +212,26 @@ __global__ __launch_bounds__(NT) void attention_values_kernel(
     const uint32_t per = div_up(P, NT);
     const uint32_t t0 = tid * per < P ? tid * per : P;
     const uint32_t nt = t0 + per < P ? per : P - t0;
-    if (tid == 0) {
-        flags_s = todo_s = 0;
-        own_s = owns_slot(ticket);
-    }
-    __syncthreads();
-    const bool own = own_s;
-    float sc[kTerms];
-    if (own) {
-        const float *src = slot_scores[ticket % kSlots] + static_cast<uint64_t>(head) * P + t0;
+    bool stale = ticket == 0;
+    if (!stale) {
 #pragma unroll
         for (uint32_t i = 0; i < kTerms; ++i)
-            if (i < nt) sc[i] = src[i];
+            if (i * NT + tid < P) {
+                pr[i * NT + tid] = __builtin_bit_cast(float, static_cast<uint32_t>(raw[i]));
+                stale |= static_cast<uint32_t>(raw[i] >> 32) != ticket;
+            }
+    }
+    stale = __any(stale);
+    if (lane == 0) stale_s[wave] = stale;
+    if (tid == 0) flags_s = todo_s = 0;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < kWaves; ++i) stale |= stale_s[i];
+    float sc[kTerms];
+    if (!stale) {
+#pragma unroll
+        for (uint32_t i = 0; i < kTerms; ++i)
+            if (i < nt) sc[i] = pr[t0 + i];
     } else {
         for (uint32_t j = tid; j < D; j += NT) qs[j] = static_cast<double>(q[static_cast<uint64_t>(head) * D + j]);
         __syncthreads();
@@ -255,11 +265,6 @@ __global__ __launch_bounds__(NT) void attention_values_kernel(
     const double incl = wave_scan(local);
     if (lane == 63) red_sum[wave] = incl;
     __syncthreads();
-    // every score of the head has reached its thread: the slot is read. (What
-    // takes it next starts after the exchange, so counting orders nothing: a
-    // release here would write back the L2.)
-    if (own && tid == 0 && atomicAdd(&slots[ticket % kSlots].done, 1u) + 1 == total)
-        atomicExch(&slots[ticket % kSlots].owner, 0u);
     if (flags_s & 1u) {
         if (tid == 0 && slice == 0) atomicOr(status, STATUS_NONFINITE_SCORE);
         if (tid < 4 && col < D)
@@ -421,7 +426,7 @@ size_t values_lds_bytes(uint32_t positions, uint32_t threads) {
     return ((static_cast<size_t>(positions) * 8 + 15) & ~static_cast<size_t>(15)) + (threads / 4 + kGroupPad) * kSliceDims * 12;
 }
 
-// Never 0; a call's slot is its ticket modulo kSlots.
+// A call's ticket: never 0, and its slot modulo kSlots.
 uint32_t next_ticket() {
     static std::atomic<uint32_t> counter{0};
     uint32_t t;
@@ -443,7 +448,7 @@ int attention_decode(const float *q, const float *kv, uint64_t row_stride, uint3
         return FMX_ERR_SHAPE_MISMATCH;
     const uint32_t group = heads / kv_heads;
     const uint32_t total = heads * div_up(head_dim, kSliceDims);
-    const bool split = positions > kSplitPositions && static_cast<uint64_t>(heads) * positions <= kSlotFloats &&
+    const bool split = positions > kSplitPositions && static_cast<uint64_t>(heads) * positions <= kSlotScores &&
                        kv_heads <= 65535;
     const uint32_t ticket = split ? next_ticket() : 0;
     // as few terms per thread as the threads allow: their exponentials and
@@ -454,7 +459,7 @@ int attention_decode(const float *q, const float *kv, uint64_t row_stride, uint3
     const uint32_t threads = positions <= 256 ? 256 : 1024;
     const size_t lds = values_lds_bytes(positions, threads);
     if (int rc = allow_lds(reinterpret_cast<const void *>(values), lds)) return rc;
-    hipLaunchKernelGGL(attention_begin_kernel, dim3(1), dim3(1), 0, s, status, ticket);
+    hipLaunchKernelGGL(attention_clear_kernel, dim3(1), dim3(1), 0, s, status);
     FMX_LAUNCH_CHECK();
     if (split) {
         const size_t tile = kScorePos * (head_dim + 4) * sizeof(float) + kScoreHeads * (head_dim + 2) * sizeof(double);

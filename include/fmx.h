@@ -18,7 +18,9 @@
  *   - Argument checks run on the host before anything is launched.
  *   - The library never allocates behind the caller's back on a compute call:
  *     scratch memory comes in through a workspace argument sized by the
- *     matching *_workspace_bytes() query.
+ *     matching *_workspace_bytes() query. (Device arrays of fixed size inside
+ *     the library: fmx_moe_decode_static's workspace, fmx_attention_decode's
+ *     scores.)
  *
  * Weight layouts
  *   Raw      GGUF blocks, row-major [rows x cols] (gguf.cpp:58-106 geometry).
@@ -283,7 +285,12 @@ int fmx_moe_bucket(const uint32_t *ids, uint32_t tokens, uint32_t top_k, uint32_
  * libm's). heads % kv_heads == 0, head_dim <= 256 and % 4 == 0, positions
  * <= 8192, pointers 16-byte aligned. workspace (>= 256 bytes): its first
  * word receives the error word; a non-finite score (INTERNAL_ERROR in the
- * engine) is reported by fmx_moe_status on it. */
+ * engine) is reported by fmx_moe_status on it. The scores pass between the
+ * call's kernels in device memory inside the library (16 MiB per GPU, four
+ * buffers taken in turn, held until the process ends). Calls may overlap in
+ * any number, captured ones and several executions of one capture included:
+ * one that finds another's scores in its buffer computes them again, which
+ * takes longer and gives the same result. */
 int fmx_attention_decode(const float *q, const float *kv, uint64_t row_stride, uint32_t v_offset,
                          uint32_t heads, uint32_t kv_heads, uint32_t head_dim, uint32_t positions,
                          double scale, float *out, void *workspace, uint64_t workspace_bytes, void *stream);

@@ -150,8 +150,8 @@ def test_attention_decode_keeps_the_ordered_sums(gpu, name, spread):
 
 
 def test_attention_decode_calls_in_flight_share_no_scores(gpu):
-    """More calls in flight than the library holds score buffers, on streams
-    of their own, each with its own inputs and workspace."""
+    """Twelve calls on streams of their own, each with its own inputs and
+    workspace (as many run at once as the process has hardware queues)."""
     import torch
     heads, kvh, D, P = 8, 2, 64, 1500
     calls = []
@@ -210,3 +210,97 @@ def test_attention_decode_captured_and_replayed(gpu):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager), f"replay {i}"
+
+
+class _Captured:
+    """Long calls of one shape, each captured on its own (its ticket is fixed
+    there), with its own inputs and workspace, to be run at once."""
+    heads, kvh, D, P = 32, 8, 128, 8192
+
+    def __init__(self, gpu, n):
+        import ctypes
+        import torch
+        self.hip, self.calls, self.execs = ctypes.CDLL("libamdhip64.so.7"), [], []
+        for i in range(n):
+            g = torch.Generator(device=gpu).manual_seed(300 + i)
+            c = dict(q=torch.randn(self.heads * self.D, generator=g, device=gpu),
+                     kv=torch.randn(self.P, 2 * self.kvh * self.D, generator=g, device=gpu),
+                     ws=torch.zeros(256, dtype=torch.uint8, device=gpu), out=torch.empty(self.heads * self.D, device=gpu))
+            self.run(c)
+            torch.cuda.synchronize()
+            self.calls.append(dict(c, want=c["out"].clone()))
+
+    def run(self, c):
+        fmx.call("fmx_attention_decode", c["q"].data_ptr(), c["kv"].data_ptr(), 2 * self.kvh * self.D, self.kvh * self.D,
+                 self.heads, self.kvh, self.D, self.P, 0.125, c["out"].data_ptr(), c["ws"].data_ptr(), 256,
+                 fmx.stream_handle())
+
+    def capture(self, c):
+        import torch
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph):
+            self.run(c)
+        return graph
+
+    def instantiate(self, graph):
+        import ctypes
+        e = ctypes.c_void_p()
+        assert self.hip.hipGraphInstantiate(ctypes.byref(e), ctypes.c_void_p(graph.raw_cuda_graph()), None, None,
+                                            ctypes.c_size_t(0)) == 0
+        self.execs.append(e)
+        return e
+
+    def together(self, *execs):
+        """Runs the instantiated graphs on a stream each, let go at once by an
+        event behind a pause, and checks every call's output."""
+        import ctypes
+        import torch
+        for c in self.calls:
+            c["out"].copy_(c["want"])
+        for c, _ in execs:
+            c["out"].zero_()
+        torch.cuda.synchronize()
+        go, gate, streams = torch.cuda.Event(), torch.cuda.Stream(), [torch.cuda.Stream() for _ in execs]
+        with torch.cuda.stream(gate):
+            torch.cuda._sleep(2_000_000)
+            go.record()
+        for (_, e), s in zip(execs, streams):
+            s.wait_event(go)
+            assert self.hip.hipGraphLaunch(e, ctypes.c_void_p(s.cuda_stream)) == 0
+        torch.cuda.synchronize()
+        for i, c in enumerate(self.calls):
+            assert torch.equal(c["out"], c["want"]), i
+
+    def close(self):
+        for e in self.execs:
+            assert self.hip.hipGraphExecDestroy(e) == 0
+
+
+@pytest.mark.parametrize("between", range(8))
+def test_attention_decode_two_calls_meet_in_one_score_buffer(gpu, between):
+    """Two long calls at once, `between` other calls apart: for some of those
+    both write the same score buffer, and each value workgroup that finds the
+    other's scores there forms its own."""
+    k = _Captured(gpu, 2)
+    a, b = k.calls
+    graphs = [k.capture(a)] + [k.capture(a) for _ in range(between)] + [k.capture(b)]
+    ea, eb = k.instantiate(graphs[0]), k.instantiate(graphs[-1])
+    for _ in range(4):
+        k.together((a, ea), (b, eb))
+        k.together((b, eb), (a, ea))
+    k.close()
+
+
+@pytest.mark.parametrize("between", range(8))
+def test_attention_decode_one_capture_twice_at_once(gpu, between):
+    """One captured call instantiated twice and both run at once, beside a
+    third call `between` calls later. The two executions share a ticket and
+    all their memory; neither disturbs the third."""
+    k = _Captured(gpu, 2)
+    a, b = k.calls
+    graphs = [k.capture(a)] + [k.capture(a) for _ in range(between)] + [k.capture(b)]
+    e1, e2, eb = k.instantiate(graphs[0]), k.instantiate(graphs[0]), k.instantiate(graphs[-1])
+    for _ in range(4):
+        k.together((a, e1), (a, e2), (b, eb))
+        k.together((a, e1), (b, eb), (a, e2))
+    k.close()

@@ -34,6 +34,7 @@ namespace fmx {
 
 namespace {
 
+constexpr uint32_t kCus = 256;
 constexpr uint32_t kMaxHeadDim = 256;
 constexpr uint32_t kMaxPositions = 8192;
 constexpr uint32_t kScorePos = 32;  // positions of a score workgroup
@@ -42,8 +43,8 @@ constexpr uint32_t kSliceDims = 16; // output elements of a value workgroup
 constexpr uint32_t kGroupPad = 4;   // its LDS rows of group sums: the four columns' stores on other banks
 
 // Up to this many positions every slice's workgroup computes the scores of its
-// head itself, one per thread: 32 heads of 128 over 256 positions 11.7 against
-// 15.3 us with the score kernel's launch before it (at 512, two per thread,
+// head itself, one per thread: 32 heads of 128 over 256 positions 11.4 us, over
+// 257, with the score kernel's launch before it, 14.4 (at 512, two per thread,
 // no faster).
 constexpr uint32_t kSplitPositions = 256;
 
@@ -422,8 +423,88 @@ __global__ __launch_bounds__(NT) void attention_values_kernel(
     }
 }
 
+// A head's whole attention on one workgroup, every sum in order: a launch with
+// nothing repeated between workgroups (attention_values_kernel repeats the
+// softmax in every slice, and its 1024 threads have a CU to themselves).
+// grid: heads; LDS: positions doubles, then as many floats.
+constexpr uint32_t kHeadThreads = 256;
+__global__ __launch_bounds__(kHeadThreads) void attention_heads_kernel(
+    const float *__restrict__ q, const float *__restrict__ kv, uint64_t row_stride, uint32_t v_offset, uint32_t group,
+    uint32_t head_dim, uint32_t positions, double scale, float *__restrict__ out, uint32_t *__restrict__ status) {
+    constexpr uint32_t kWaves = kHeadThreads / 64;
+    extern __shared__ __align__(16) char lds[];
+    __shared__ __align__(16) double qs[kMaxHeadDim];
+    __shared__ float red_max[kWaves];
+    __shared__ bool bad_s[kWaves];
+    __shared__ double sum_s;
+    const uint32_t tid = threadIdx.x, wave = tid >> 6, head = blockIdx.x, P = positions, D = head_dim;
+    double *ex = reinterpret_cast<double *>(lds);
+    float *pr = reinterpret_cast<float *>(ex + P);
+    const float *keys = kv + static_cast<uint64_t>(head / group) * D;
+    float *o = out + static_cast<uint64_t>(head) * D;
+    if (tid < D) qs[tid] = static_cast<double>(q[static_cast<uint64_t>(head) * D + tid]);
+    __syncthreads();
+    float m = -__builtin_inff();
+    bool bad = false;
+    for (uint32_t t = tid; t < P; t += kHeadThreads) {
+        const float s = static_cast<float>(dot_in_order(keys + t * row_stride, qs, D) * scale);
+        bad |= !__builtin_isfinite(s);
+        m = fmaxf(m, s);
+        pr[t] = s;
+    }
+    for (uint32_t d = 32; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
+    bad = __any(bad);
+    if ((tid & 63) == 0) {
+        red_max[wave] = m;
+        bad_s[wave] = bad;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < kWaves; ++i) {
+        m = fmaxf(m, red_max[i]);
+        bad |= bad_s[i];
+    }
+    if (bad) {
+        if (tid == 0) atomicOr(status, STATUS_NONFINITE_SCORE);
+        if (tid < D) o[tid] = 0.0f;
+        return;
+    }
+    const double md = static_cast<double>(m);
+    for (uint32_t t = tid; t < P; t += kHeadThreads) ex[t] = exp(static_cast<double>(pr[t]) - md);
+    __syncthreads();
+    if (tid == 0) sum_s = add_in_order(ex, P, 0.0);
+    __syncthreads();
+    const double sum = sum_s;
+    for (uint32_t t = tid; t < P; t += kHeadThreads) pr[t] = static_cast<float>(ex[t] / sum);
+    __syncthreads();
+    if (tid >= D) return;
+    const float *v = keys + v_offset + tid;
+    double acc = 0.0; // fma: the product is exact
+#pragma unroll 8
+    for (uint32_t t = 0; t < P; ++t)
+        acc = fma(static_cast<double>(pr[t]), static_cast<double>(v[t * row_stride]), acc);
+    o[tid] = static_cast<float>(acc);
+}
+
 size_t values_lds_bytes(uint32_t positions, uint32_t threads) {
     return ((static_cast<size_t>(positions) * 8 + 15) & ~static_cast<size_t>(15)) + (threads / 4 + kGroupPad) * kSliceDims * 12;
+}
+
+// Whether a call of `total` slices takes attention_heads_kernel. A slice's
+// workgroup of 1024 threads fills a CU: up to 256 slices run at once, and only
+// the shortest caches are better off on one workgroup per head; beyond, the
+// slices come in rounds while the heads do not. Heads x kv heads x dim x
+// positions, heads kernel / slices, us: 32 x 4 x 128 x 16 7.1 / 8.9, x 64 8.5 /
+// 9.0, x 96 9.6 / 9.2; 64 x 64 x 128 x 256 15.0 / 16.2, x 400 21.7 / 23.6, x 512
+// 28.9 / 25.1; 128 x 128 x 256 x 256 26 / 68, x 1024 96 / 127, x 1536 192 / 176.
+// Where the scores do not fit a buffer every slice forms its head's: 256 x 32 x
+// 128 x 3000 191 / 469, but 128 x 128 x 128 x 8192 (1024 slices) about 1100 /
+// 760. Over 1800 such calls the rule's choice never costs more than 21% over
+// the other's time.
+bool attention_on_heads(uint32_t heads, uint32_t total, uint32_t positions) {
+    if (total <= kCus) return positions < 72;
+    if (positions > kSplitPositions && static_cast<uint64_t>(heads) * positions > kSlotScores) return total > 1024;
+    return positions < 450 || positions < total * 11 / 20;
 }
 
 // A call's ticket: never 0, and its slot modulo kSlots.
@@ -448,6 +529,16 @@ int attention_decode(const float *q, const float *kv, uint64_t row_stride, uint3
         return FMX_ERR_SHAPE_MISMATCH;
     const uint32_t group = heads / kv_heads;
     const uint32_t total = heads * div_up(head_dim, kSliceDims);
+    if (attention_on_heads(heads, total, positions)) {
+        const size_t lds = static_cast<size_t>(positions) * 12;
+        if (int rc = allow_lds(reinterpret_cast<const void *>(attention_heads_kernel), lds)) return rc;
+        hipLaunchKernelGGL(attention_clear_kernel, dim3(1), dim3(1), 0, s, status);
+        FMX_LAUNCH_CHECK();
+        hipLaunchKernelGGL(attention_heads_kernel, dim3(heads), dim3(kHeadThreads), lds, s, q, kv, row_stride, v_offset,
+                           group, head_dim, positions, scale, out, status);
+        FMX_LAUNCH_CHECK();
+        return FMX_OK;
+    }
     const bool split = positions > kSplitPositions && static_cast<uint64_t>(heads) * positions <= kSlotScores &&
                        kv_heads <= 65535;
     const uint32_t ticket = split ? next_ticket() : 0;

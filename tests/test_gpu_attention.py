@@ -100,6 +100,15 @@ ORDERED = {
     "mqa_6_of_1x256_4099": (6, 1, 256, 4099),
     "longest_8192": (32, 32, 128, 8192),
     "beyond_the_slot": (72, 8, 64, 8192),
+    # one workgroup per head and either side of that rule: the shortest caches,
+    # more slices than CUs, more scores than a buffer holds
+    "heads_71": (4, 2, 64, 71),
+    "slices_72": (4, 2, 64, 72),
+    "heads_260_slices": (65, 65, 64, 449),
+    "slices_260_slices": (65, 65, 64, 450),
+    "heads_ragged_dim": (180, 2, 100, 691),
+    "slices_ragged_dim": (180, 2, 100, 693),
+    "heads_beyond_the_slot": (260, 4, 64, 2100),
 }
 
 

@@ -169,18 +169,29 @@ int launch_matvec(const PackedGeometry &g, const void *packed, const float *x, f
     return FMX_OK;
 }
 
-// The pair kernel's twice as many wavefronts with seven chunks each in flight
-// serve the matrices whose rows leave the device short of them. [4096 x 4096]
-// matvec_kernel -> pair: Q4_0 14.2 -> 7.2, Q8_0 18.3 -> 7.2, Q4_K 11.8 -> 8.5
-// us; [4096 x 14336] 44.9 -> 13.5, 58.2 -> 18.6, 34.5 -> 20.9. Past max_rows its
-// 17% more instructions per block cost more: Q4_0 [14336 x 4096] 14.9 -> 11.6
-// but [32000 x 4096] 18.9 -> 19.5; Q8_0 there 30.6 -> 27.2; Q4_K [14336 x 4096]
-// 16.8 -> 19.4. (15 chunks in flight: the same up to 4096 rows, slower above.)
+// Rows up to which the pair kernel serves a type: its twice as many wavefronts
+// with seven chunks each in flight are for matrices whose rows leave the device
+// short of them. [4096 x 4096] matvec_kernel -> pair: Q4_0 14.2 -> 7.2, Q8_0
+// 18.3 -> 7.2, Q4_K 11.8 -> 8.5 us; [4096 x 14336] 44.9 -> 13.5, 58.2 -> 18.6,
+// 34.5 -> 20.9. With more rows its 17% more instructions per block cost more,
+// and sooner the shorter the rows, whose chains are short anyway (GPU time):
+// Q4_0 [16384 x 4096] 14.5 -> 11.3, [32000 x 4096] 18.9 -> 19.5, [16384 x 512]
+// 4.0 -> 4.2, [8192 x 256] 0.93 of it and [10240 x 256] 1.05; Q8_0 [32768 x 4096]
+// 29.5 -> 26.9 but [32768 x 2048] 15.4 -> 16.8 and x 512 5.5 -> 7.1; Q4_K, the
+// most per block, [4096 x 2048] 6.7 -> 5.1, [8192 x 2048] 7.2 -> 7.7, x 8192 21.5
+// -> 19.8. (15 chunks in flight: the same up to 4096 rows, slower above.)
+uint32_t pair_rows(uint32_t type_id, uint32_t cols) {
+    if (type_id == FMX_TYPE_Q4_K) return cols >= 8192 ? 8192 : 4096;
+    if (cols < 1024) return cols < 512 ? 8192 : 12288;
+    if (type_id == FMX_TYPE_Q4_0 || cols < 2048) return 16384;
+    return cols < 4096 ? 24576 : 32768;
+}
+
 template <class P, int NR>
-int launch_matvec_quant(uint32_t max_rows, const PackedGeometry &g, const void *packed, const float *x, float *y, hipStream_t s) {
+int launch_matvec_quant(const PackedGeometry &g, const void *packed, const float *x, float *y, hipStream_t s) {
     using T = typename P::T;
     const size_t lds = static_cast<size_t>(g.blocks) * T::kLdsFloatsPerBlock * sizeof(float);
-    if (g.rows > max_rows || g.blocks % T::kPerChunk != 0 || lds > kMatvecMaxLds)
+    if (g.rows > pair_rows(T::kType, g.blocks * T::kBlock) || g.blocks % T::kPerChunk != 0 || lds > kMatvecMaxLds)
         return launch_matvec<T, NR>(g, packed, x, y, s);
     auto k = matvec_pair_kernel<P, 7>;
     if (int rc = allow_lds(reinterpret_cast<const void *>(k), lds)) return rc;
@@ -219,9 +230,9 @@ extern "C" int fmx_matvec(uint32_t type_id, const void *packed, const float *x, 
                                static_cast<const float *>(packed), x, y, out_dim, in_dim);
         FMX_LAUNCH_CHECK();
         return FMX_OK;
-    case FMX_TYPE_Q4_0: return launch_matvec_quant<PairQ40, 2>(16384, g, packed, x, y, s);
-    case FMX_TYPE_Q8_0: return launch_matvec_quant<PairQ80, 2>(32768, g, packed, x, y, s);
-    case FMX_TYPE_Q4_K: return launch_matvec_quant<PairQ4K, 1>(8192, g, packed, x, y, s);
+    case FMX_TYPE_Q4_0: return launch_matvec_quant<PairQ40, 2>(g, packed, x, y, s);
+    case FMX_TYPE_Q8_0: return launch_matvec_quant<PairQ80, 2>(g, packed, x, y, s);
+    case FMX_TYPE_Q4_K: return launch_matvec_quant<PairQ4K, 1>(g, packed, x, y, s);
     case FMX_TYPE_Q6_K: {
         // quads per row: as many as give every SIMD eight wavefronts. Every
         // workgroup stages x, and long inputs let few share a CU's LDS: there

@@ -177,7 +177,9 @@ def test_gemm_quant_errors(gpu):
     (8, 3, 33792),
     (12, 1, 256), (12, 17, 1792), (12, 16, 2048), (12, 15, 2304), (12, 33, 4352), (12, 4, 16384), (12, 3, 33792),
     # either side of the rows each type's two-group kernel serves
-    (2, 16384, 256), (2, 16385, 256), (8, 32768, 128), (8, 32769, 128), (12, 8192, 256), (12, 8193, 256)])
+    (2, 16384, 256), (2, 16385, 256), (8, 32768, 128), (8, 32769, 128), (12, 8192, 256), (12, 8193, 256),
+    (2, 8192, 256), (2, 8193, 256), (2, 12289, 512), (2, 16385, 1024), (8, 8193, 256), (8, 12288, 512), (8, 12289, 512),
+    (8, 16385, 1024), (8, 24576, 2048), (8, 24577, 2048), (12, 4096, 256), (12, 4097, 256), (12, 4097, 8192)])
 def test_matvec_two_groups_per_row_bitwise(gpu, t, rows, cols):
     test_matvec_bitwise_vs_oracle(gpu, t, rows, cols)
 

@@ -18,8 +18,9 @@ namespace {
 
 constexpr uint32_t kThreads = 256;              // 4 wavefronts
 constexpr uint32_t kLdsBudgetFloats = 8 * 1024; // 32 KiB of x per tile
-constexpr size_t kMatvecMaxLds = 128 * 1024;     // the Q6_K kernel's x and dots
-constexpr uint32_t kQ6Quads = 131072;
+constexpr size_t kMatvecMaxLds = 128 * 1024;     // the pair kernel's x
+constexpr size_t kQ6MaxLds = 159 * 1024;         // the Q6_K quad kernel's x and dots
+constexpr uint32_t kQ6Quads = 131072;            // eight wavefronts per SIMD
 
 template <class T, int NR>
 __global__ __launch_bounds__(kThreads) void matvec_kernel(
@@ -119,6 +120,22 @@ __global__ __launch_bounds__(kThreads) void matvec_q6_k_kernel(const uint8_t *__
     if (c == 0 && r < rows) y[r] = total;
 }
 
+// Q6_K, four 16-lane groups per row, group g taking blocks g, g + 4, ..., x from
+// memory; the block dots meet in LDS (4 rows x blocks) and one lane adds them in
+// block order from 0, as q6_k_row_chains does.
+__global__ __launch_bounds__(kThreads) void matvec_q6_k_split_kernel(const uint8_t *__restrict__ w,
+                                                                     const float *__restrict__ x,
+                                                                     float *__restrict__ y, uint32_t rows,
+                                                                     uint32_t blocks) {
+    extern __shared__ __align__(16) float q6_lds[];
+    constexpr uint32_t kRows = kThreads / 64;
+    const uint32_t tid = threadIdx.x, lr = tid >> 6, r0 = blockIdx.x * kRows;
+    const uint8_t *row = w + static_cast<uint64_t>(r0 + lr < rows ? r0 + lr : rows - 1) * blocks * 210;
+    q6_k_block_dots(row, x, blocks, (tid >> 4) & 3, 4, tid & 15, q6_lds + lr * blocks);
+    __syncthreads();
+    if (tid < kRows && r0 + tid < rows) y[r0 + tid] = q6_sum_dots(q6_lds + tid * blocks, blocks);
+}
+
 // Q6_K with x in LDS (block b at xs + b * kQ6XStride): a quad of lanes works on
 // one block at a time (Q6Quad), G quads per row, quad g taking blocks g,
 // g + G, ... (each block's dot is independent); the block dots meet in LDS and
@@ -145,13 +162,85 @@ __global__ __launch_bounds__(NT) void matvec_q6_k_quad_kernel(const uint8_t *__r
 }
 
 template <uint32_t NT, uint32_t G>
-int launch_q6_k_quad(const void *w, const float *x, float *y, uint32_t rows, uint32_t blocks, hipStream_t s) {
+int launch_q6_k_quad(const void *w, const float *x, float *y, uint32_t rows, uint32_t blocks, hipStream_t s, bool *done) {
     constexpr uint32_t kRows = NT / 4 / G;
     const size_t lds = (q6_dots_floats(kRows, blocks) + static_cast<size_t>(blocks) * kQ6XStride) * sizeof(float);
+    *done = lds <= kQ6MaxLds;
+    if (!*done) return FMX_OK;
     auto k = matvec_q6_k_quad_kernel<NT, G>;
     if (int rc = allow_lds(reinterpret_cast<const void *>(k), lds)) return rc;
     hipLaunchKernelGGL(k, dim3(div_up(rows, kRows)), dim3(NT), lds, s, static_cast<const uint8_t *>(w), x, y,
                        rows, blocks);
+    FMX_LAUNCH_CHECK();
+    return FMX_OK;
+}
+
+// The quad kernel's layout for a Q6_K matrix (*done: whether x and the dots fit
+// the LDS). Every workgroup stages x, so long rows (32 blocks and more, where
+// few workgroups of 256 threads share a CU's LDS) take larger ones; past 80
+// blocks one fills a CU, and its threads and quads are such that the device's
+// 256 workgroups hold the rows. [4096 x 8192] 8.5 us on 512 threads and 16 quads
+// a row, [6144 x 14336] 20.7 (1024 threads 27.5, x not staged 24.4), [16384 x
+// 14336] on 8 quads 40.9 (256 threads 50.3); [5120 x 27648] 1024 threads and 8
+// quads 40 (x not staged 39, one lane group a row 73), [4096 x 25088] 23 (30, 56),
+// [2048 x 24576] 512 threads and 16 quads 13.2 (18.9).
+// Shorter rows: with few rows the chain over a row's blocks bounds, as many quads
+// as it has blocks ([1024 x 1536] eight 3.5, four 4.2; up to eight blocks as long
+// as the rows leave room, [12288 x 1280] eight 6.4, two 6.8); with more, the
+// device is full and quads without a block are lost: the most quads that leave
+// at most a fifth idle ([8192 x 5120] 16, 8, 4 quads 12.9, 11.3, 10.4; [4096 x 2560] 5.4,
+// 5.6, 5.3; [16384 x 2560] eight 13.1, four 11.1).
+int launch_q6_k_quads(const void *w, const float *x, float *y, uint32_t rows, uint32_t blocks, hipStream_t s, bool *done) {
+    const uint32_t want = kQ6Quads / rows; // quads per row that fill the device
+    if (blocks > 80 && rows > 1024) {
+        if (rows <= 2048) return launch_q6_k_quad<512, 16>(w, x, y, rows, blocks, s, done);
+        if (rows <= 4096) return launch_q6_k_quad<1024, 16>(w, x, y, rows, blocks, s, done);
+        if (rows <= 8192) return launch_q6_k_quad<1024, 8>(w, x, y, rows, blocks, s, done);
+        return launch_q6_k_quad<512, 8>(w, x, y, rows, blocks, s, done);
+    }
+    if (blocks >= 32 && rows >= 4096 && want >= 8)
+        return want >= 16 ? launch_q6_k_quad<512, 16>(w, x, y, rows, blocks, s, done)
+                          : launch_q6_k_quad<512, 8>(w, x, y, rows, blocks, s, done);
+    uint32_t g = 16;
+    if (blocks <= 8 ? want > 8 : blocks <= 16 ? want >= 32 : want >= 128)
+        while (g / 2 >= blocks) g /= 2;
+    else
+        while (g > 1 && (g > want || 4 * div_up(blocks, g) * g > 5 * blocks)) g /= 2;
+    switch (g) {
+    case 16: return launch_q6_k_quad<256, 16>(w, x, y, rows, blocks, s, done);
+    case 8: return launch_q6_k_quad<256, 8>(w, x, y, rows, blocks, s, done);
+    case 4: return launch_q6_k_quad<256, 4>(w, x, y, rows, blocks, s, done);
+    case 2: return launch_q6_k_quad<256, 2>(w, x, y, rows, blocks, s, done);
+    }
+    return launch_q6_k_quad<256, 1>(w, x, y, rows, blocks, s, done);
+}
+
+// Q6_K: the quads, but x staged and the dots joined cost more than they save
+// where a row is over at once (GPU time): up to three blocks on 16 lanes
+// ([4096 x 512] 2.6 us, quads 3.4; [12288 x 768] 4.5, 4.5), and with few rows
+// where the quads' second round is mostly idle or their one round long, on four
+// groups of 16 lanes ([1024 x 2048] 2.9, quads 3.5; x 3072 3.4, 3.6; x 5120 4.4,
+// 4.7; but x 4096 3.8, 3.6). x past the LDS: four groups below 8192 rows
+// ([1024 x 28672] 15 us, one group 49), one from there ([8192 x 28672] 74, two
+// 138).
+int launch_matvec_q6_k(const void *w, const float *x, float *y, uint32_t rows, uint32_t blocks, hipStream_t s) {
+    const uint8_t *wb = static_cast<const uint8_t *>(w);
+    auto split = [&]() -> int {
+        hipLaunchKernelGGL(matvec_q6_k_split_kernel, dim3(div_up(rows, kThreads / 64)), dim3(kThreads),
+                           kThreads / 64 * blocks * sizeof(float), s, wb, x, y, rows, blocks);
+        FMX_LAUNCH_CHECK();
+        return FMX_OK;
+    };
+    const bool one = blocks <= 3 && rows <= (blocks == 1 ? 32768 : 12288);
+    if (!one) {
+        if (rows <= 1024 && ((blocks >= 8 && blocks <= 12) || (blocks >= 17 && blocks <= 20))) return split();
+        bool done;
+        if (int rc = launch_q6_k_quads(w, x, y, rows, blocks, s, &done)) return rc;
+        if (done) return FMX_OK;
+        if (rows < 8192 && blocks <= 4096) return split(); // (64 KiB of dots)
+    }
+    hipLaunchKernelGGL(matvec_q6_k_kernel, dim3(div_up(rows, kThreads / 16)), dim3(kThreads), 0, s, wb, x, y, rows,
+                       blocks);
     FMX_LAUNCH_CHECK();
     return FMX_OK;
 }
@@ -233,31 +322,7 @@ extern "C" int fmx_matvec(uint32_t type_id, const void *packed, const float *x, 
     case FMX_TYPE_Q4_0: return launch_matvec_quant<PairQ40, 2>(g, packed, x, y, s);
     case FMX_TYPE_Q8_0: return launch_matvec_quant<PairQ80, 2>(g, packed, x, y, s);
     case FMX_TYPE_Q4_K: return launch_matvec_quant<PairQ4K, 1>(g, packed, x, y, s);
-    case FMX_TYPE_Q6_K: {
-        // quads per row: as many as give every SIMD eight wavefronts. Every
-        // workgroup stages x, and long inputs let few share a CU's LDS: there
-        // a row's many quads come in larger workgroups, where the rows fill
-        // the device with them ([4096 x 14336] 18.9 -> 16.2 us; [8000 x 4096]
-        // 8.4 -> 11.3)
-        const size_t with_x = (q6_dots_floats(64, g.blocks) + static_cast<size_t>(g.blocks) * kQ6XStride) * 4;
-        if (with_x <= kMatvecMaxLds) {
-            const uint32_t want = kQ6Quads / out_dim;
-            const bool wide = g.blocks >= 32 && out_dim >= 4096;
-            if (want >= 16 && g.blocks >= 16)
-                return wide ? launch_q6_k_quad<1024, 16>(packed, x, y, out_dim, g.blocks, s)
-                            : launch_q6_k_quad<256, 16>(packed, x, y, out_dim, g.blocks, s);
-            if (want >= 8 && g.blocks >= 8)
-                return wide ? launch_q6_k_quad<512, 8>(packed, x, y, out_dim, g.blocks, s)
-                            : launch_q6_k_quad<256, 8>(packed, x, y, out_dim, g.blocks, s);
-            if (want >= 4 && g.blocks >= 4) return launch_q6_k_quad<256, 4>(packed, x, y, out_dim, g.blocks, s);
-            if (want >= 2 && g.blocks >= 2) return launch_q6_k_quad<256, 2>(packed, x, y, out_dim, g.blocks, s);
-            return launch_q6_k_quad<256, 1>(packed, x, y, out_dim, g.blocks, s);
-        }
-        hipLaunchKernelGGL(matvec_q6_k_kernel, dim3(div_up(out_dim, kThreads / 16)), dim3(kThreads), 0, s,
-                           static_cast<const uint8_t *>(packed), x, y, out_dim, g.blocks);
-        FMX_LAUNCH_CHECK();
-        return FMX_OK;
-    }
+    case FMX_TYPE_Q6_K: return launch_matvec_q6_k(packed, x, y, out_dim, g.blocks, s);
     }
     return FMX_ERR_UNSUPPORTED_QUANTISATION;
 }

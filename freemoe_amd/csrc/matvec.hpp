@@ -155,6 +155,32 @@ __device__ inline float q6_k_row_chains(const uint8_t *__restrict__ row, const f
 // on different banks.
 constexpr uint32_t kQ6XStride = 272;
 
+// Dots of blocks b0, b0 + stride, ... (< blocks) of one Q6_K row on 16
+// consecutive lanes, each as in q6_k_row_chains (chain c over elements
+// 16 m + c, the lanes' chains joined), x from memory, the next block's share
+// requested before a block's chain runs; lane 0 writes block b's dot to out[b].
+__device__ __forceinline__ void q6_k_block_dots(const uint8_t *__restrict__ row, const float *__restrict__ x,
+                                                uint32_t blocks, uint32_t b0, uint32_t stride, uint32_t c,
+                                                float *out) {
+    Q6Lane q[2];
+    auto load = [&](uint32_t u, uint32_t b) {
+        q[u].load(row + static_cast<uint64_t>(b) * 210, x + static_cast<uint64_t>(b) * 256, c);
+    };
+    if (b0 < blocks) load(0, b0);
+    for (uint32_t b = b0; b < blocks; b += 2 * stride) {
+#pragma unroll
+        for (uint32_t u = 0; u < 2; ++u) {
+            const uint32_t bu = b + u * stride;
+            if (bu >= blocks) break;
+            if (bu + stride < blocks) load(u ^ 1, bu + stride);
+            const float acc = q[u].chain();
+            const float t = acc + lane_xor<8>(acc);
+            const float dot = hsum8_first(t); // exact in every lane, as above
+            if (c == 0) out[bu] = dot;
+        }
+    }
+}
+
 // A quad's share of a raw Q6_K block: lane i of four consecutive lanes owns
 // chains 4 i .. 4 i + 3, whose quants lie side by side, so that the fields of
 // four elements come out of each word at a time (285 VALU instructions for 64

@@ -190,6 +190,12 @@ def test_matvec_two_groups_per_row_bitwise(gpu, t, rows, cols):
     # rows, and inputs past the LDS (16 lanes a row)
     (131073, 256), (65537, 512), (65536, 512), (40000, 256), (32769, 1024), (32768, 1024), (16385, 2048), (16384, 2048),
     (16383, 1792), (8193, 4096), (8192, 4096), (8191, 3840), (5, 4096), (1, 256), (3, 768), (4099, 8192), (4095, 8192),
-    (9001, 8192), (7, 29440), (5, 30208), (3, 33792)])
+    (9001, 8192), (7, 29440), (5, 30208), (3, 33792),
+    # each line of the choice: up to three blocks on 16 lanes, four groups of 16
+    # lanes, quads by rows and idle share, the layouts of long rows, x past the LDS
+    (32768, 256), (32769, 256), (12288, 768), (12289, 768), (64, 1024), (1024, 2048), (1025, 2048), (513, 3072),
+    (1023, 3328), (9, 4352), (1024, 5120), (1000, 5376), (4096, 1280), (4097, 1280), (8193, 2560), (5121, 8192),
+    (1025, 20736), (2049, 20736), (4097, 20736), (8193, 20736), (1025, 20480), (1000, 24832), (6, 37376), (5, 37888),
+    (1027, 37120), (1030, 37376)])
 def test_matvec_q6_k_quads_bitwise(gpu, rows, cols):
     test_matvec_bitwise_vs_oracle(gpu, 14, rows, cols)

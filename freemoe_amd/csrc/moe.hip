@@ -1353,16 +1353,16 @@ __global__ __launch_bounds__(kThreads) void gate_up_q6_k_quad_kernel(ExpertArgs 
 }
 
 // Q6_K down rows on quads of lanes, G per row, every rank's activations in
-// LDS; NT / 4 / G slots, NT / 4 / G / top_k rows of every rank per workgroup,
+// LDS, with kTiled `tile` blocks of each at a time (block dots are independent
+// and meet in LDS; the loop costs the others 2 to 4%); NT / 4 / G slots, NT / 4 / G / top_k rows of every rank per workgroup,
 // then the combine in rank order and the residual. LDS: NT / 4 / G slots x
 // blocks dots, then the activations.
-template <uint32_t NT, uint32_t G>
+template <uint32_t NT, uint32_t G, bool kTiled>
 __global__ __launch_bounds__(NT) void down_q6_k_quad_kernel(ExpertArgs a, const float *__restrict__ x,
-                                                                        const float *__restrict__ act,
-                                                                        const uint32_t *__restrict__ ids,
-                                                                        const float *__restrict__ w,
-                                                                        float *__restrict__ out,
-                                                                        uint32_t *__restrict__ status) {
+                                                            const float *__restrict__ act,
+                                                            const uint32_t *__restrict__ ids,
+                                                            const float *__restrict__ w, float *__restrict__ out,
+                                                            uint32_t *__restrict__ status, uint32_t tile) {
     extern __shared__ __align__(16) float q6_lds[];
     constexpr uint32_t kSlots = NT / 4 / G;
     __shared__ float dres[kSlots];
@@ -1379,10 +1379,23 @@ __global__ __launch_bounds__(NT) void down_q6_k_quad_kernel(ExpertArgs a, const 
     }
     const uint8_t *row = static_cast<const uint8_t *>(a.down[e]) + static_cast<uint64_t>(j < H ? j : H - 1) * blocks * 210;
     Q6Quad first;
-    first.load(row + (part < blocks ? part : 0) * 210, i);
-    q6_stage_x(act, K * F, xs, tid, NT);
-    __syncthreads();
-    q6_quad_block_dots(first, row, xs + rank * blocks * kQ6XStride, blocks, part, G, i, dots + slot * blocks);
+    if constexpr (kTiled) {
+        for (uint32_t b0 = 0; b0 < blocks; b0 += tile) {
+            const uint32_t nb = blocks - b0 < tile ? blocks - b0 : tile;
+            const uint8_t *from = row + static_cast<uint64_t>(b0) * 210;
+            first.load(from + (part < nb ? part : 0) * 210, i);
+            if (b0) __syncthreads(); // the tile before is read
+            for (uint32_t r = 0; r < K; ++r)
+                q6_stage_x(act + static_cast<uint64_t>(r) * F + b0 * 256, nb * 256, xs + r * nb * kQ6XStride, tid, NT);
+            __syncthreads();
+            q6_quad_block_dots(first, from, xs + rank * nb * kQ6XStride, nb, part, G, i, dots + slot * blocks + b0);
+        }
+    } else {
+        first.load(row + (part < blocks ? part : 0) * 210, i);
+        q6_stage_x(act, K * F, xs, tid, NT); // the ranks' activations: one run of memory
+        __syncthreads();
+        q6_quad_block_dots(first, row, xs + rank * blocks * kQ6XStride, blocks, part, G, i, dots + slot * blocks);
+    }
     __syncthreads();
     if (tid < K * jpw) // slot tid: rank tid / jpw
         dres[tid] = ids[tid / jpw] >= a.experts ? 0.0f : q6_sum_dots(dots + tid * blocks, blocks);
@@ -1519,37 +1532,53 @@ int launch_gate_up(const ExpertArgs &a, const float *h, const float *logits, uin
 
 template <uint32_t NT, uint32_t G>
 int launch_down_q6_k(const ExpertArgs &a, const float *x, const float *act, const uint32_t *ids, const float *w,
-                     float *out, uint32_t *status, size_t lds, hipStream_t s, const hipEvent_t *kev) {
-    auto k = down_q6_k_quad_kernel<NT, G>;
+                     float *out, uint32_t *status, uint32_t tile, size_t lds, hipStream_t s, const hipEvent_t *kev) {
+    auto k = tile * 256 < a.ffn ? down_q6_k_quad_kernel<NT, G, true> : down_q6_k_quad_kernel<NT, G, false>;
     if (int rc = allow_lds(reinterpret_cast<const void *>(k), lds)) return rc;
     const dim3 grid(div_up(a.hidden, NT / 4 / G / a.top_k));
     if (kev)
-        hipExtLaunchKernelGGL(k, grid, dim3(NT), lds, s, kev[0], kev[1], 0, a, x, act, ids, w, out, status);
+        hipExtLaunchKernelGGL(k, grid, dim3(NT), lds, s, kev[0], kev[1], 0, a, x, act, ids, w, out, status, tile);
     else
-        hipLaunchKernelGGL(k, grid, dim3(NT), lds, s, a, x, act, ids, w, out, status);
+        hipLaunchKernelGGL(k, grid, dim3(NT), lds, s, a, x, act, ids, w, out, status, tile);
     FMX_LAUNCH_CHECK();
     return FMX_OK;
 }
 
-// Q6_K down rows on quads, where every rank's activations fit the LDS
-// (*done: whether they do). A workgroup per CU takes hidden / 256 rows of
-// every rank; its quads, 64 or 256, go to as many blocks of a row at once as
-// there are (at most 16).
+// Q6_K down rows on quads (*done: whether they took them). A workgroup per CU
+// takes hidden / 256 rows of every rank, on the fewest threads whose quads hold
+// as many blocks of a row at once as there are (at most 16); few rows of 9 to 15
+// blocks take all 16 ((1536, 2304, 2) 6.3 us, on eight quads 9.4).
+// Short rows whose block count leaves quads idle stay on 16 lanes while the
+// device is not full of them (layers (hidden, ffn, top-k), kernel us, 16 lanes /
+// quads: (1024, 768, 6) 4.4 / 8.9, (2048, 768, 8) 5.9 / 9.0, (1536, 1536, 2) 4.8 /
+// 8.4, (2560, 1536, 8) 11.6 / 13.0; but (5120, 1536, 6) 22.1 / 15.2, (4096, 1280,
+// 8) 14.0 / 13.9, and four blocks, (2048, 1024, 6), 7.5 / 7.1).
 int launch_down_q6_k(const ExpertArgs &a, const float *x, const float *act, const uint32_t *ids, const float *w,
                      float *out, uint32_t *status, hipStream_t s, const hipEvent_t *kev, bool *done) {
     const uint32_t slots = div_up(a.hidden, kCus) * a.top_k, blocks = a.ffn / 256;
-    const bool small = slots * (blocks < 16 ? blocks : 16) <= 64;
-    const uint32_t quads = small ? 64 : 256;
-    uint32_t G = 16;
-    while (G > 2 && (G > blocks || G * slots > quads)) G /= 2;
-    const size_t lds =
-        (q6_dots_floats(quads / G, blocks) + static_cast<size_t>(a.top_k) * blocks * kQ6XStride) * sizeof(float);
-    *done = a.top_k <= quads / G && lds <= kMaxLds - 2048;
-    if (!*done) return FMX_OK;
+    *done = false;
+    if (blocks < 8 && (blocks & (blocks - 1)) && static_cast<uint64_t>(a.hidden) * a.top_k * blocks <= 128 * 1024)
+        return FMX_OK;
+    uint32_t G = 16, quads = 128;
+    if (blocks <= 8 || blocks >= 16 || slots > 16 || a.top_k > 8) { // (sixteen quads of such a row in one round)
+        while (G > 2 && G > blocks) G /= 2;
+        quads = slots * G <= 64 ? 64 : slots * G <= 128 ? 128 : 256;
+        while (G > 2 && G * slots > quads) G /= 2;
+    }
+    const uint32_t dots = q6_dots_floats(quads / G, blocks), room = (kMaxLds - 2048) / sizeof(float);
+    if (a.top_k > quads / G || dots >= room) return FMX_OK;
+    // all blocks of the activations, or as many whole rounds of the quads as fit
+    uint32_t tile = (room - dots) / (a.top_k * kQ6XStride);
+    if (tile >= blocks) tile = blocks;
+    else if (tile >= G) tile = div_up(div_up(blocks, div_up(blocks, tile / G * G)), G) * G;
+    else return FMX_OK;
+    *done = true;
+    const size_t lds = (dots + static_cast<size_t>(a.top_k) * tile * kQ6XStride) * sizeof(float);
     auto pick = [&](auto g) {
         constexpr uint32_t kG = decltype(g)::value;
-        return small ? launch_down_q6_k<256, kG>(a, x, act, ids, w, out, status, lds, s, kev)
-                     : launch_down_q6_k<1024, kG>(a, x, act, ids, w, out, status, lds, s, kev);
+        return quads == 64    ? launch_down_q6_k<256, kG>(a, x, act, ids, w, out, status, tile, lds, s, kev)
+               : quads == 128 ? launch_down_q6_k<512, kG>(a, x, act, ids, w, out, status, tile, lds, s, kev)
+                              : launch_down_q6_k<1024, kG>(a, x, act, ids, w, out, status, tile, lds, s, kev);
     };
     switch (G) {
     case 16: return pick(std::integral_constant<uint32_t, 16>());

@@ -648,6 +648,19 @@ def test_decode_q6_k_quads(gpu, H, F, E, K):
     assert check_layer(gpu, lw, wl.inputs(H, 2, 92)) == 0
 
 
+@pytest.mark.parametrize("H,F,E,K", [
+    # Q6_K down: short rows of 3, 5, 6 and 7 blocks on 16 lanes and, with more
+    # rows, on quads; 9 to 15 blocks on sixteen quads; 256, 512 and 1024 threads
+    (1024, 768, 10, 6), (2816, 768, 18, 16), (512, 1280, 6, 4), (1536, 1536, 4, 2), (4864, 1792, 5, 4), (1536, 2304, 4, 2),
+    (256, 3840, 3, 2), (768, 4096, 4, 2), (1024, 2048, 6, 4), (2048, 2816, 6, 4),
+    # activations past the LDS, in tiles: the last one full, ragged, of less
+    # than a round; too many ranks for one round (16 lanes)
+    (512, 9984, 5, 4), (256, 14336, 5, 4), (512, 5120, 9, 8), (1024, 16384, 5, 4), (4096, 9216, 5, 4), (256, 18432, 17, 16)])
+def test_decode_q6_k_down_layouts(gpu, H, F, E, K):
+    lw = wl.make_layer(H, F, E, K, wl.Q6_K, 93 + H + F)
+    assert check_layer(gpu, lw, wl.inputs(H, 2, 94)) == 0
+
+
 @pytest.mark.parametrize("H", [4064, 4128, 6176, 16384])
 def test_rmsnorm_sum_interval_ragged_hidden(gpu, H):
     """The bounded ordered sum between the certificate and the replay, where a

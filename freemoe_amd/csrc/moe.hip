@@ -516,21 +516,29 @@ __device__ __attribute__((noinline)) double ordered_sum(const double *a, uint32_
 }
 
 // sum(a_j) as ordered_sum's (n <= 16 NT, a in LDS), to within `doubt`. Every
-// thread calls it and gets both. Out of line, as ordered_sum.
+// thread calls it and gets both. Out of line, as ordered_sum. With 1024 threads
+// the terms are read twice instead of held: 16 of them beside the caller's
+// values spilled (rmsnorm_kernel<1024, 4> 6 registers, route_rows_kernel<1024>
+// 12 more).
 struct SumInterval {
     double sum, doubt;
 };
 template <uint32_t NT>
 __device__ __attribute__((noinline)) SumInterval ordered_sum_interval(const double *a, uint32_t n) {
-    constexpr uint32_t kWaves = NT / 64;
+    constexpr uint32_t kWaves = NT / 64, kHeld = NT > 256 ? 1 : 16;
     __shared__ double red[3][kWaves], part[kWaves];
     const uint32_t tid = threadIdx.x, wave = tid >> 6, c = div_up(n, NT);
     const uint32_t t0 = tid * c < n ? tid * c : n, nt = n - t0 < c ? n - t0 : c;
-    double x[16], local = 0.0;
+    double x[kHeld], local = 0.0;
+    if constexpr (kHeld == 1) {
+#pragma unroll 4
+        for (uint32_t i = 0; i < nt; ++i) local += a[t0 + i];
+    } else {
 #pragma unroll
-    for (uint32_t i = 0; i < 16; ++i) {
-        x[i] = i < nt ? a[t0 + i] : 0.0;
-        local += x[i];
+        for (uint32_t i = 0; i < kHeld; ++i) {
+            x[i] = i < nt ? a[t0 + i] : 0.0;
+            local += x[i];
+        }
     }
     const double incl = wave_scan(local);
     if ((tid & 63) == 63) part[wave] = incl;
@@ -544,7 +552,15 @@ __device__ __attribute__((noinline)) SumInterval ordered_sum_interval(const doub
     // (an ordered prefix sum is off by at most n 2^-53 of the whole, run by
     // 38 2^-53; n <= 2^14)
     SumInterval r;
-    ordered_interval(x, nt, run, all * 0x1p-37, red, r.sum, r.doubt);
+    const double margin = all * 0x1p-37;
+    if constexpr (kHeld == 1) {
+        OrderedInterval s{run, margin};
+#pragma unroll 2
+        for (uint32_t i = 0; i < nt; ++i) s.add(a[t0 + i]);
+        s.total(red, r.sum, r.doubt);
+    } else {
+        ordered_interval(x, nt, run, margin, red, r.sum, r.doubt);
+    }
     return r;
 }
 

@@ -54,64 +54,78 @@ __device__ __forceinline__ void add_exact(double &hi, double &lo, double v, doub
 }
 
 // The sum of a workgroup's terms in order, s_t = rn(s_t-1 + x_t) from 0, to
-// within `doubt`: thread i holds the nt <= kTerms terms after thread i - 1's
-// and the (unordered) sum `run` of those before, which no ordered prefix sum
-// is further from than `margin`. While s stays in one binade, of unit u, a
-// step adds x_t rounded to a multiple of u, whatever s is, but for exact ties;
-// so where the margin leaves no doubt about the binades of s_t-1 and s_t, the
+// within `doubt`: thread i adds the terms after thread i - 1's, from the
+// (unordered) sum `run` of those before, which no ordered prefix sum is
+// further from than `margin`. While s stays in one binade, of unit u, a step
+// adds x_t rounded to a multiple of u, whatever s is, but for exact ties; so
+// where the margin leaves no doubt about the binades of s_t-1 and s_t, the
 // step is known but for half a unit at a tie, and elsewhere to within a unit.
-// Every thread returns the same sum; red: 3 x kWaves doubles of LDS. x_t has
-// at most 48 significant bits or is no larger in magnitude than s_t.
+// x_t has at most 48 significant bits or is no larger in magnitude than s_t.
+struct OrderedInterval {
+    double run, margin;
+    double hi = 0.0, lo = 0.0, unc = 0.0;
+
+    __device__ __forceinline__ void add(double x) {
+        const double after = run + x;
+        const uint32_t k = exponent_of(fabs(after) + margin);
+        const double u = power_of(k > 52 ? k - 52 : 0);
+        double r = x;
+        if (exponent_of(fabs(after) - margin) != k || fabs(run) <= margin || exponent_of(fabs(run) - margin) < k) {
+            unc += u;
+        } else if (fabs(x) < power_of(k)) { // else a multiple of u
+            const double big = copysign(power_of(k), x);
+            r = (big + x) - big;
+            if (fabs(x - r) * 2.0 == u) {
+                r = x;
+                unc += 0.5 * u;
+            }
+        }
+        add_exact(hi, lo, r);
+        run = after;
+    }
+
+    // After the thread's last term. Every thread returns the same sum; red: 3 x
+    // kWaves doubles of LDS.
+    template <uint32_t kWaves>
+    __device__ __forceinline__ void total(double (&red)[3][kWaves], double &sum, double &doubt) {
+        auto wave_total = [&] {
+            add_exact(hi, lo, dpp_or_zero<0x111, 0xF>(hi), dpp_or_zero<0x111, 0xF>(lo));
+            add_exact(hi, lo, dpp_or_zero<0x112, 0xF>(hi), dpp_or_zero<0x112, 0xF>(lo));
+            add_exact(hi, lo, dpp_or_zero<0x114, 0xF>(hi), dpp_or_zero<0x114, 0xF>(lo));
+            add_exact(hi, lo, dpp_or_zero<0x118, 0xF>(hi), dpp_or_zero<0x118, 0xF>(lo));
+            add_exact(hi, lo, dpp_or_zero<0x142, 0xA>(hi), dpp_or_zero<0x142, 0xA>(lo));
+            add_exact(hi, lo, dpp_or_zero<0x143, 0xC>(hi), dpp_or_zero<0x143, 0xC>(lo));
+            hi = last_lane(hi);
+            lo = last_lane(lo);
+            unc = wave_sum(unc);
+        };
+        wave_total();
+        const uint32_t lane = threadIdx.x & 63;
+        if (lane == 0) {
+            red[0][threadIdx.x >> 6] = hi;
+            red[1][threadIdx.x >> 6] = lo;
+            red[2][threadIdx.x >> 6] = unc;
+        }
+        __syncthreads();
+        hi = lane < kWaves ? red[0][lane] : 0.0;
+        lo = lane < kWaves ? red[1][lane] : 0.0;
+        unc = lane < kWaves ? red[2][lane] : 0.0;
+        wave_total();
+        sum = hi + lo;
+        // the bound's own roundings, and the sum's
+        doubt = unc * 1.0009765625 + fabs(sum) * 0x1p-52 + margin * 0x1p-40;
+    }
+};
+
+// OrderedInterval over the first nt <= kTerms of a thread's terms.
 template <uint32_t kTerms, uint32_t kWaves>
 __device__ __forceinline__ void ordered_interval(const double (&x)[kTerms], uint32_t nt, double run, double margin,
                                                  double (&red)[3][kWaves], double &sum, double &doubt) {
-    double hi = 0.0, lo = 0.0, unc = 0.0;
+    OrderedInterval s{run, margin};
 #pragma unroll
     for (uint32_t i = 0; i < kTerms; ++i)
-        if (i < nt) {
-            const double after = run + x[i];
-            const uint32_t k = exponent_of(fabs(after) + margin);
-            const double u = power_of(k > 52 ? k - 52 : 0);
-            double r = x[i];
-            if (exponent_of(fabs(after) - margin) != k || fabs(run) <= margin || exponent_of(fabs(run) - margin) < k) {
-                unc += u;
-            } else if (fabs(x[i]) < power_of(k)) { // else a multiple of u
-                const double big = copysign(power_of(k), x[i]);
-                r = (big + x[i]) - big;
-                if (fabs(x[i] - r) * 2.0 == u) {
-                    r = x[i];
-                    unc += 0.5 * u;
-                }
-            }
-            add_exact(hi, lo, r);
-            run = after;
-        }
-    auto wave_total = [&] {
-        add_exact(hi, lo, dpp_or_zero<0x111, 0xF>(hi), dpp_or_zero<0x111, 0xF>(lo));
-        add_exact(hi, lo, dpp_or_zero<0x112, 0xF>(hi), dpp_or_zero<0x112, 0xF>(lo));
-        add_exact(hi, lo, dpp_or_zero<0x114, 0xF>(hi), dpp_or_zero<0x114, 0xF>(lo));
-        add_exact(hi, lo, dpp_or_zero<0x118, 0xF>(hi), dpp_or_zero<0x118, 0xF>(lo));
-        add_exact(hi, lo, dpp_or_zero<0x142, 0xA>(hi), dpp_or_zero<0x142, 0xA>(lo));
-        add_exact(hi, lo, dpp_or_zero<0x143, 0xC>(hi), dpp_or_zero<0x143, 0xC>(lo));
-        hi = last_lane(hi);
-        lo = last_lane(lo);
-        unc = wave_sum(unc);
-    };
-    wave_total();
-    const uint32_t lane = threadIdx.x & 63;
-    if (lane == 0) {
-        red[0][threadIdx.x >> 6] = hi;
-        red[1][threadIdx.x >> 6] = lo;
-        red[2][threadIdx.x >> 6] = unc;
-    }
-    __syncthreads();
-    hi = lane < kWaves ? red[0][lane] : 0.0;
-    lo = lane < kWaves ? red[1][lane] : 0.0;
-    unc = lane < kWaves ? red[2][lane] : 0.0;
-    wave_total();
-    sum = hi + lo;
-    // the bound's own roundings, and the sum's
-    doubt = unc * 1.0009765625 + fabs(sum) * 0x1p-52 + margin * 0x1p-40;
+        if (i < nt) s.add(x[i]);
+    s.total(red, sum, doubt);
 }
 
 } // namespace

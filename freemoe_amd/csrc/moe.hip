@@ -1478,12 +1478,16 @@ int launch_gate_up_q(const ExpertArgs &a, const float *h, const float *logits, u
     // top-k), gate_up_kernel -> split, us per token: (4096, 4096, 2) Q4_0 29.5
     // -> 26.0, Q8_0 38.6 -> 34.2, Q4_K 47.0 -> 40.3; (2048, 1024, 8) Q4_K 39.1
     // -> 35.5; past that (2048, 5632, 2) the same, (4096, 14336, 2) 52.7 ->
-    // 57.5. Q4_K, whose chains are the longest, also stays on one
-    // gate_up_kernel workgroup per CU where the split leaves some CUs two:
-    // (2048, 768, 8) 34.9 -> 36.2, against 28.6 -> 28.1 for Q4_0.
+    // 57.5. Q4_K rows of more chunks than a wavefront has in flight also stay
+    // on one gate_up_kernel workgroup per CU where the split leaves some CUs
+    // two: their chains are the longest, and two of them on a SIMD take turns.
+    // Kernel time of the split over gate_up_kernel's, 16 such (ffn, top-k) from
+    // (768, 6) to (7168, 1): hidden 2048 0.99 to 1.10, 4096 1.02 to 1.08, but
+    // 1792 (7 chunks) 0.88 to 0.91, 1024 0.92 to 0.99; Q4_0 of hidden 2048 0.95
+    // to 1.05, 4096 0.88 to 0.94, Q8_0 0.87 to 0.95 and 0.78 to 0.91.
     const uint32_t whole = div_up(a.ffn, kThreads / 64 * 7) * a.top_k, split = div_up(a.ffn, kThreads / 16) * a.top_k;
     if (split <= 2 * kCus && a.gu_tile >= a.gu.blocks &&
-        !(TG::kType == FMX_TYPE_Q4_K && whole <= kCus && split > kCus)) {
+        !(TG::kType == FMX_TYPE_Q4_K && a.gu.blocks > kSplitPF && whole <= kCus && split > kCus)) {
         auto gu = gate_up_split_kernel<TG, kSplitPF>;
         if (int rc = allow_lds(reinterpret_cast<const void *>(gu), lds)) return rc;
         return launch_timed(gu, dim3(div_up(a.ffn, kThreads / 16), a.top_k), lds, s, kev, a, h, logits, ids, w,

@@ -621,6 +621,14 @@ def test_decode_split_gate_up_and_batched_down_staging(gpu, H, F, E, K, t):
     assert check_layer(gpu, lw, wl.inputs(H, 2, 62)) == 0
 
 
+@pytest.mark.parametrize("H", [1792, 2048])
+def test_decode_split_gate_up_q4_k_chunks_in_flight(gpu, H):
+    """Q4_K gate and up rows of as many chunks as a wavefront has in flight and
+    of one more, where the split leaves some CUs two workgroups."""
+    lw = wl.make_layer(H, 2304, 3, 2, wl.Q4_K, 61 + H)
+    assert check_layer(gpu, lw, wl.inputs(H, 2, 62)) == 0
+
+
 def test_decode_clears_the_error_word(gpu):
     """A stale error word is zeroed by the call itself, for one and several
     tokens and for a block-type router (whose RMSNorm is a launch of its own)."""

@@ -1262,11 +1262,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1),
     }
 }
 
-// F32 and Q6_K experts: 16 lanes per row (RowDot16: F32 in gemv_avx2_row's
-// order, Q6_K in row_dot_fused_scalar's), h staged in LDS first (every row
-// of the workgroup reads all of it; the groups of a wavefront read the same
-// elements at once). LDS: hidden floats.
-template <uint32_t kT>
+// F32 gate and up rows: 16 lanes per row in gemv_avx2_row's order, h staged in
+// LDS first (every row of the workgroup reads all of it; the groups of a
+// wavefront read the same elements at once). LDS: hidden floats.
 __global__ __launch_bounds__(kThreads) void gate_up_rows16_kernel(ExpertArgs a, const float *__restrict__ h,
                                                                   const float *__restrict__ logits,
                                                                   uint32_t *__restrict__ ids, float *__restrict__ w,
@@ -1286,14 +1284,15 @@ __global__ __launch_bounds__(kThreads) void gate_up_rows16_kernel(ExpertArgs a, 
     __syncthreads();
     const uint32_t j = blockIdx.x * (kThreads / 16) + (tid >> 4);
     const uint32_t jr = j < F ? j : F - 1;
-    const float g = RowDot16<kT>::dot(a.gate[e], jr, hl16, H, c);
-    const float u = RowDot16<kT>::dot(a.up[e], jr, hl16, H, c);
+    const float g = RowDot16<FMX_TYPE_F32>::dot(a.gate[e], jr, hl16, H, c);
+    const float u = RowDot16<FMX_TYPE_F32>::dot(a.up[e], jr, hl16, H, c);
     if (c == 0 && j < F) act[static_cast<uint64_t>(rank) * F + j] = swiglu(g, u);
 }
 
-// F32 and Q6_K down rows on 16 lanes each (RowDot16), then the combine in
-// rank order and the residual, as down_kernel; 16 slots, 16 / top_k rows of
-// every rank per workgroup.
+// Down rows on 16 lanes each (RowDot16: F32 in gemv_avx2_row's order, the Q6_K
+// rows that launch_down_q6_k leaves in row_dot_fused_scalar's), then the
+// combine in rank order and the residual, as down_kernel; 16 slots, 16 / top_k
+// rows of every rank per workgroup.
 template <uint32_t kT>
 __global__ __launch_bounds__(kThreads) void down_rows16_kernel(ExpertArgs a, const float *__restrict__ x,
                                                                const float *__restrict__ act,
@@ -1539,7 +1538,7 @@ int launch_gate_up(const ExpertArgs &a, const float *h, const float *logits, uin
     const dim3 grid16(div_up(a.ffn, kThreads / 16), a.top_k);
     switch (a.type_gu) {
     case FMX_TYPE_F32:
-        return launch_timed(gate_up_rows16_kernel<FMX_TYPE_F32>, grid16, a.hidden * sizeof(float), s, kev, a, h, logits,
+        return launch_timed(gate_up_rows16_kernel, grid16, a.hidden * sizeof(float), s, kev, a, h, logits,
                             ids, w, act, status);
     case FMX_TYPE_Q6_K:
         return launch_gate_up_q6_k(a, h, logits, ids, w, act, status, s, kev);

@@ -956,8 +956,9 @@ int launch_gemm(K k, dim3 grid, uint32_t threads, size_t lds, hipStream_t s, hip
 }
 
 // Whether a GEMM of block type T takes the few-row kernels: a token's experts
-// are distinct, so up to 64 tokens no tile has more rows (Q6_K's raw blocks
-// have no 64-byte runs of a row's K step to put on four lanes).
+// are distinct, so up to 64 tokens no tile has more rows. Their quarter of a
+// chunk is laid out for the packed types; Q6_K's raw blocks, read in place,
+// have none yet.
 template <class T>
 bool few_rows(const PrefillBuffers &b) {
     return !std::is_same_v<T, GQ6K> && b.tokens <= kSmallRows;
@@ -981,7 +982,8 @@ int launch_gemms(const ExpertArgs &a, const PrefillBuffers &b, uint32_t max_tile
         return rc;
     }
     hipEvent_t *dev = kev ? kev + 2 : nullptr;
-    // (the K splits start at whole chunks there)
+    // there the K splits start at whole chunks: two steps of Q4_0 and Q4_K (of
+    // Q8_0 one, whose odd splits could take them as well)
     if (few_rows<TD>(b) && (b.splits == 1 || steps % 2 == 0)) {
         if constexpr (!std::is_same_v<TD, GQ6K>)
             return launch_gemm(small_down_kernel<TD>, dim3(a.hidden / 128, b.splits, max_tiles), kSThreads,

@@ -20,8 +20,8 @@
 // the sum in position order can lie from the parallel one. A probability or
 // an output whose float is the same over that whole interval is the engine's;
 // where one is not, one lane adds the terms in order. For 32 heads of 128 over
-// 8 kv heads and 2000 positions (16 MB of cache: 3 us of HBM) a call takes 19
-// us, three dependent launches (traced one by one: 1, 5-6 and 12-13 us), each a
+// 8 kv heads and 2000 positions (16 MB of cache: 3 us of HBM) a call takes 20
+// us, three dependent launches (traced one by one: 1, 6 and 14 us), each a
 // chain of memory, LDS and double-precision latencies; walking every sum in
 // order on one workgroup per head took 215 us (32 of the 256 CUs in use). 8192
 // positions: 46 us, 83 over 32 kv heads.
